@@ -8,9 +8,9 @@
 // Layout and kernels. Every intermediate is an FP32 plane in one arena, per
 // pair and scale: 47 planes of w x h (rows packed, planes 64-float aligned).
 // The reference runs about 60 launches per scale, each a full pass over one
-// or two planes; here one scale is six launches, each a 2-D tile kernel that
-// stages its input with halo in LDS and fuses everything pointwise around
-// its stencil:
+// or two planes; here a stage is one launch of a 2-D tile kernel that stages
+// its input with halo in LDS and fuses everything pointwise around its
+// stencil:
 //
 //   opsin   sigma 1.2 blur of linear RGB + opsin dynamics       -> XYB
 //   low     sigma 7.156 blur of XYB                             -> low band
@@ -25,9 +25,9 @@
 //           map and the norm partial sums                        -> map, partials
 //
 // Both images of a pair run in one launch (grid z = pair x image), and a
-// batch of pairs in the same launches. The half scale runs first, so that
-// the full scale's mask kernel blends and reduces in its own pass.
-// Separable blurs divide each pass by the sum of the taps that fall inside
+// batch of pairs in the same launches; so do both scales, but for the mask:
+// there the half scale runs first, so that the full scale's kernel blends and
+// reduces in its own pass. Separable blurs divide each pass by the sum of the taps that fall inside
 // the image, as the reference does (gaussianblur.hpp:55-85): the per-column
 // and per-row factors come from the running tap sums.
 #include "butter.hpp"
@@ -105,16 +105,18 @@ __device__ __forceinline__ float at(const float* base, int off) {
     return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (uint64_t)((uint32_t)off * 4u));
 }
 
-// Tile of this workgroup, XCD-aware: hardware workgroup b (in launch order
-// x fastest, then y, then z) runs on XCD b % 8, so tiles are numbered such
-// that each XCD takes one contiguous range of tile rows, and the halos that
-// neighbouring tiles share are read through that XCD's L2 once.
+__host__ __device__ constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+// Tile (x, y) of plane set z.
 struct TileIdx {
     int x, y, z;
 };
-__device__ __forceinline__ TileIdx tile_of_block() {
-    const int nx = gridDim.x, ny = gridDim.y, nz = gridDim.z;
-    const int b = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
+
+// Tile of workgroup b of nx * ny * nz (x fastest, then y, then z),
+// XCD-aware: hardware workgroup b runs on XCD b % 8, so tiles are numbered
+// such that each XCD takes one contiguous range of tile rows, and the halos
+// that neighbouring tiles share are read through that XCD's L2 once.
+__device__ __forceinline__ TileIdx tile_of(int b, int nx, int ny, int nz) {
     const int v = xcd_block(b, nx * ny * nz);
     // the divisions run on the vector unit; the tile is the workgroup's, so
     // it is moved to scalar registers, and the plane addresses built from it
@@ -124,6 +126,35 @@ __device__ __forceinline__ TileIdx tile_of_block() {
     t.y = __builtin_amdgcn_readfirstlane((v / nx) % ny);
     t.z = __builtin_amdgcn_readfirstlane(v / (nx * ny));
     return t;
+}
+
+// Tile of this workgroup in a grid of one scale.
+__device__ __forceinline__ TileIdx tile_of_block() {
+    return tile_of(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z);
+}
+
+// A stage that runs both scales in one launch: the workgroups of the full
+// scale come first, then those of the half scale, whose tiles fill the
+// launch's tail. No stage up to the mask reads the other scale's planes. A
+// launch of each scale by itself leaves most of the GPU idle where the
+// picture is small (a 256 x 256 pair has 64 tiles of the blurs, 16 in the half
+// scale) and pays a start and a tail of its own: 207 -> 133 us for one
+// 256 x 256 pair, 477 -> 430 us for one 1920 x 1080 pair, 5.41 -> 5.34 ms for
+// sixteen, all with the same results.
+struct Scales {
+    Scale s[2];
+};
+
+// Scale and tile of this workgroup of a two-scale launch with tiles of
+// TW x TH and nz plane sets; leaves the scale in S.
+template <int TW, int TH>
+__device__ __forceinline__ TileIdx tile_of_scales(const Scales& SS, int nz, Scale& S) {
+    const int nx0 = cdiv(SS.s[0].w, TW), ny0 = cdiv(SS.s[0].h, TH);
+    const int n0 = nx0 * ny0 * nz;
+    const bool half = (int)blockIdx.x >= n0;
+    S = half ? SS.s[1] : SS.s[0];
+    return half ? tile_of(blockIdx.x - n0, cdiv(SS.s[1].w, TW), cdiv(SS.s[1].h, TH), nz)
+                : tile_of(blockIdx.x, nx0, ny0, nz);
 }
 
 // 1 / (sum of the taps inside [0, n)) at position p in [0, n) for a window of
@@ -666,12 +697,13 @@ __device__ __forceinline__ void blur_tile(BlurLds<R>& L, BlurRegs<R>& S, const f
 }
 
 // sigma 1.2 blur of linear RGB + opsin dynamics (colors.hpp:50-91) -> XYB
-__global__ __launch_bounds__(kThreads) void butter_opsin_kernel(Scale S, const Taps* __restrict__ taps,
+__global__ __launch_bounds__(kThreads) void butter_opsin_kernel(Scales SS, int nz, const Taps* __restrict__ taps,
                                                                 float intensity) {
     constexpr int R = kRad[SG_OPSIN];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_OPSIN;
-    const TileIdx ti = tile_of_block();
+    Scale S;
+    const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
     const int pair = ti.z >> 1, im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     edge_factors<R, kTW, kTH>(L.colf, L.rowf, T, S.w, S.h, ox0, oy0);
@@ -713,11 +745,12 @@ __global__ __launch_bounds__(kThreads) void butter_opsin_kernel(Scale S, const T
 
 // sigma 7.156 blur: low band (stored as values, XybLowFreqToVals) and the
 // residual XYB - low (separatefrequencies.hpp:142-170)
-__global__ __launch_bounds__(kThreads) void butter_low_kernel(Scale S, const Taps* __restrict__ taps) {
+__global__ __launch_bounds__(kThreads) void butter_low_kernel(Scales SS, int nz, const Taps* __restrict__ taps) {
     constexpr int R = kRad[SG_LOW];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_LOW;
-    const TileIdx ti = tile_of_block();
+    Scale S;
+    const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
     const int pair = ti.z >> 1, im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     const RunPos p = run_pos();
@@ -752,11 +785,12 @@ __global__ __launch_bounds__(kThreads) void butter_low_kernel(Scale S, const Tap
 // sigma 3.225 blur of the residual: middle band after its range operation,
 // high residual = residual - middle band, X's residual suppressed by Y's
 // (separatefrequencies.hpp:160-189)
-__global__ __launch_bounds__(kThreads) void butter_mid_kernel(Scale S, const Taps* __restrict__ taps) {
+__global__ __launch_bounds__(kThreads) void butter_mid_kernel(Scales SS, int nz, const Taps* __restrict__ taps) {
     constexpr int R = kRad[SG_MID];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_MID;
-    const TileIdx ti = tile_of_block();
+    Scale S;
+    const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
     const int pair = ti.z >> 1, im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     const RunPos p = run_pos();
@@ -795,11 +829,12 @@ __global__ __launch_bounds__(kThreads) void butter_mid_kernel(Scale S, const Tap
 
 // sigma 1.564 blur of the high residual: high and ultra-high bands
 // (separatefrequencies.hpp:117-140, 190-200)
-__global__ __launch_bounds__(kThreads) void butter_high_kernel(Scale S, const Taps* __restrict__ taps) {
+__global__ __launch_bounds__(kThreads) void butter_high_kernel(Scales SS, int nz, const Taps* __restrict__ taps) {
     constexpr int R = kRad[SG_HIGH];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_HIGH;
-    const TileIdx ti = tile_of_block();
+    Scale S;
+    const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
     const int pair = ti.z >> 1, im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     const RunPos p = run_pos();
@@ -968,9 +1003,10 @@ __device__ __forceinline__ float l2_asym(float a, float b, float wgt, float wlt)
     return r + wlt * v * v;
 }
 
-__global__ __launch_bounds__(kThreads) void butter_diff_kernel(Scale S, DiffParams D) {
+__global__ __launch_bounds__(kThreads) void butter_diff_kernel(Scales SS, int nz, DiffParams D) {
     __shared__ float dt[kDSH * kDSW];
-    const TileIdx ti = tile_of_block();
+    Scale S;
+    const TileIdx ti = tile_of_scales<kDW, kDH>(SS, nz, S);
     const int pair = ti.z;
     const int ox0 = ti.x * kDW, oy0 = ti.y * kDH;
     const int tx = threadIdx.x & (kDW - 1), ty = threadIdx.x / kDW;
@@ -1265,8 +1301,6 @@ __global__ __launch_bounds__(kThreads) void butter_norm_kernel(const double* __r
     }
 }
 
-int cdiv(int a, int b) { return (a + b - 1) / b; }
-
 int row_pitch(int w) { return (w + 63) / 64 * 64; }
 int64_t plane_floats(int w, int h) { return (int64_t)row_pitch(w) * h; }
 
@@ -1425,34 +1459,6 @@ void Engine::launch(int fmt, int n) {
     auto mark = [&](int st) {
         if (prof) (void)hipEventRecord(ev_[st], stream_);
     };
-    // stage marks: ev_[s] before the stage's first launch; the half and full
-    // scale launches of a stage are interleaved with others, so per-stage time
-    // is taken by a second, stage-ordered pass only when profiling
-    auto scale_pass = [&](const Scale& S, bool full, int only) {
-        const dim3 blk(kThreads);
-        const dim3 gt(cdiv(S.w, kTW), cdiv(S.h, kTH), 2 * n);
-        if (only < 0 || only == ST_OPSIN) butter_opsin_kernel<<<gt, blk, 0, stream_>>>(S, taps_d_, intensity_);
-        if (only < 0 || only == ST_LOW) butter_low_kernel<<<gt, blk, 0, stream_>>>(S, taps_d_);
-        if (only < 0 || only == ST_MID) butter_mid_kernel<<<gt, blk, 0, stream_>>>(S, taps_d_);
-        if (only < 0 || only == ST_HIGH) butter_high_kernel<<<gt, blk, 0, stream_>>>(S, taps_d_);
-        if (only < 0 || only == ST_DIFF)
-            butter_diff_kernel<<<dim3(cdiv(S.w, kDW), cdiv(S.h, kDH), n), blk, 0, stream_>>>(S, D);
-        if (only < 0 || only == ST_MASK) {
-            NormArgs N;
-            N.qnorm = q_;
-            N.partials = partials_d_;
-            N.tiles = mask_tiles_;
-            N.pairs = desc_d_;
-            N.half_map_base = S1.base + (int64_t)P_MAP * S1.plane;
-            N.half_pair = S1.pair;
-            N.half_pitch = S1.pitch;
-            const dim3 gm(cdiv(S.w, kMT), cdiv(S.h, kMT), n);
-            if (full)
-                butter_mask_kernel<true><<<gm, blk, 0, stream_>>>(S, taps_d_, N);
-            else
-                butter_mask_kernel<false><<<gm, blk, 0, stream_>>>(S, taps_d_, N);
-        }
-    };
     const dim3 gi(cdiv(w2_, 16), cdiv(h2_, 16), n);
     auto input = [&] {
         if (staged420_) {
@@ -1465,30 +1471,52 @@ void Engine::launch(int fmt, int n) {
         }
         launch_input_fmt(fmt, gi, stream_, desc_d_, S0, S1, std::make_integer_sequence<int, IN_NUM_FORMATS>{});
     };
-    if (!prof) {
-        input();
-        scale_pass(S1, false, -1);
-        scale_pass(S0, true, -1);
-        butter_norm_kernel<<<dim3(n), dim3(kThreads), 0, stream_>>>(partials_d_, mask_tiles_, q_, (int64_t)w_ * h_,
-                                                                    norms_d_);
-        timed_ = false;
-    } else {
-        // stage-ordered: every stage's half- and full-scale launches back to
-        // back between two events; the data dependences hold because each
-        // stage of the half scale only reads half-scale planes
-        mark(ST_INPUT);
-        input();
-        for (int st = ST_OPSIN; st <= ST_MASK; st++) {
-            mark(st);
-            scale_pass(S1, false, st);
-            scale_pass(S0, true, st);
+    const Scales SS{{S0, S1}};
+    // workgroups of a two-scale launch with tiles of tw x th and nz plane sets
+    auto grid2 = [&](int tw, int th, int nz) {
+        return dim3((unsigned)(nz * (cdiv(S0.w, tw) * cdiv(S0.h, th) + cdiv(S1.w, tw) * cdiv(S1.h, th))));
+    };
+    auto mask = [&](const Scale& S, bool full) {
+        NormArgs N;
+        N.qnorm = q_;
+        N.partials = partials_d_;
+        N.tiles = mask_tiles_;
+        N.pairs = desc_d_;
+        N.half_map_base = S1.base + (int64_t)P_MAP * S1.plane;
+        N.half_pair = S1.pair;
+        N.half_pitch = S1.pitch;
+        const dim3 gm(cdiv(S.w, kMT), cdiv(S.h, kMT), n);
+        if (full)
+            butter_mask_kernel<true><<<gm, dim3(kThreads), 0, stream_>>>(S, taps_d_, N);
+        else
+            butter_mask_kernel<false><<<gm, dim3(kThreads), 0, stream_>>>(S, taps_d_, N);
+    };
+    auto stage = [&](int st) {
+        const dim3 blk(kThreads);
+        switch (st) {
+            case ST_INPUT: input(); break;
+            case ST_OPSIN:
+                butter_opsin_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_, intensity_);
+                break;
+            case ST_LOW: butter_low_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_); break;
+            case ST_MID: butter_mid_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_); break;
+            case ST_HIGH: butter_high_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_); break;
+            case ST_DIFF: butter_diff_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n, D); break;
+            case ST_MASK:
+                mask(S1, false);  // the full scale blends its map with this one's
+                mask(S0, true);
+                break;
+            default:
+                butter_norm_kernel<<<dim3(n), blk, 0, stream_>>>(partials_d_, mask_tiles_, q_, (int64_t)w_ * h_,
+                                                                 norms_d_);
         }
-        mark(ST_NORM);
-        butter_norm_kernel<<<dim3(n), dim3(kThreads), 0, stream_>>>(partials_d_, mask_tiles_, q_, (int64_t)w_ * h_,
-                                                                    norms_d_);
-        mark(ST_COUNT);
-        timed_ = true;
+    };
+    for (int st = 0; st < ST_COUNT; st++) {
+        mark(st);
+        stage(st);
     }
+    mark(ST_COUNT);
+    timed_ = prof;
     HIP_OR_THROW(hipGetLastError(), E_BadDeviceCode);
 }
 
