@@ -35,7 +35,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 
+#include "butter_dev.hpp"
+#include "butter_strip.hpp"
 #include "engine.hpp"  // VshipErr, HIP_OR_THROW
 #include "yuv_dev.hpp"
 
@@ -43,222 +46,6 @@ namespace vship {
 namespace bt {
 
 namespace {
-
-constexpr int kThreads = 256;
-constexpr int kSigmaCount = 5;
-// src/butter/gaussianblur.hpp:27-42: window max(floor(3 sigma), 8)
-constexpr double kSigma[kSigmaCount] = {1.2, 1.56416327805, 2.7, 3.22489901262, 7.15593339443};
-constexpr int kRad[kSigmaCount] = {8, 8, 8, 9, 21};
-enum : int { SG_OPSIN = 0, SG_HIGH = 1, SG_MASK = 2, SG_MID = 3, SG_LOW = 4 };
-
-// Work planes of one pair at one scale. Groups of three are [image][X, Y, B],
-// groups of two [image][X, Y].
-enum : int {
-    P_LIN = 0,   // linear RGB
-    P_XYB = 6,   // opsin XYB
-    P_LFV = 12,  // low band, as values
-    P_T = 18,    // XYB - low band
-    P_MF = 24,   // middle band
-    P_HFR = 30,  // high residual (before its blur)
-    P_HF = 34,   // high band
-    P_UHF = 38,  // ultra-high band
-    P_ACS = 42,  // AC sum (all channels) without the mask term
-    P_DCS = 43,  // DC sum
-    P_M0 = 44,   // mask input of the reference image
-    P_M1 = 45,   // mask input of the distorted image
-    P_MAP = 46,  // distortion map (half scale)
-    P_COUNT = 47
-};
-
-struct Scale {
-    float* base;
-    int w, h;
-    int pitch;      // floats between rows (a multiple of 64)
-    int64_t plane;  // floats between planes
-    int64_t pair;   // floats between pairs
-};
-
-__device__ __forceinline__ float* plane_of(const Scale& S, int pair, int p) {
-    return S.base + (int64_t)pair * S.pair + (int64_t)p * S.plane;
-}
-
-// plane_of for a pair and plane that are the same for the whole workgroup,
-// held in scalar registers: without the read-first-lane the compiler folds
-// the plane offset into every per-lane address as 64-bit vector arithmetic
-// (the offset, not the pointer, goes through it, so that the pointer stays
-// derived from the kernel argument and its loads stay global, not flat)
-__device__ __forceinline__ float* plane_u(const Scale& S, int pair, int p) {
-    const uint64_t v = (uint64_t)((int64_t)pair * S.pair + (int64_t)p * S.plane);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return S.base + (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
-// Element off of a plane whose base is the same for the whole workgroup: a
-// 32-bit byte offset from that base, which the compiler emits as the
-// scalar-base + 32-bit vector-offset address form, with no 64-bit vector
-// address arithmetic. Planes hold fewer than 2^30 floats (the engine checks).
-__device__ __forceinline__ float& at(float* base, int off) {
-    return *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + (uint64_t)((uint32_t)off * 4u));
-}
-__device__ __forceinline__ float at(const float* base, int off) {
-    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (uint64_t)((uint32_t)off * 4u));
-}
-
-__host__ __device__ constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
-
-// Tile (x, y) of plane set z.
-struct TileIdx {
-    int x, y, z;
-};
-
-// Tile of workgroup b of nx * ny * nz (x fastest, then y, then z),
-// XCD-aware: hardware workgroup b runs on XCD b % 8, so tiles are numbered
-// such that each XCD takes one contiguous range of tile rows, and the halos
-// that neighbouring tiles share are read through that XCD's L2 once.
-__device__ __forceinline__ TileIdx tile_of(int b, int nx, int ny, int nz) {
-    const int v = xcd_block(b, nx * ny * nz);
-    // the divisions run on the vector unit; the tile is the workgroup's, so
-    // it is moved to scalar registers, and the plane addresses built from it
-    // stay scalar
-    TileIdx t;
-    t.x = __builtin_amdgcn_readfirstlane(v % nx);
-    t.y = __builtin_amdgcn_readfirstlane((v / nx) % ny);
-    t.z = __builtin_amdgcn_readfirstlane(v / (nx * ny));
-    return t;
-}
-
-// Tile of this workgroup in a grid of one scale.
-__device__ __forceinline__ TileIdx tile_of_block() {
-    return tile_of(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z);
-}
-
-// A stage that runs both scales in one launch: the workgroups of the full
-// scale come first, then those of the half scale, whose tiles fill the
-// launch's tail. No stage up to the mask reads the other scale's planes. A
-// launch of each scale by itself leaves most of the GPU idle where the
-// picture is small (a 256 x 256 pair has 64 tiles of the blurs, 16 in the half
-// scale) and pays a start and a tail of its own: 207 -> 133 us for one
-// 256 x 256 pair, 477 -> 430 us for one 1920 x 1080 pair, 5.41 -> 5.34 ms for
-// sixteen, all with the same results.
-struct Scales {
-    Scale s[2];
-};
-
-// Scale and tile of this workgroup of a two-scale launch with tiles of
-// TW x TH and nz plane sets; leaves the scale in S.
-template <int TW, int TH>
-__device__ __forceinline__ TileIdx tile_of_scales(const Scales& SS, int nz, Scale& S) {
-    const int nx0 = cdiv(SS.s[0].w, TW), ny0 = cdiv(SS.s[0].h, TH);
-    const int n0 = nx0 * ny0 * nz;
-    const bool half = (int)blockIdx.x >= n0;
-    S = half ? SS.s[1] : SS.s[0];
-    return half ? tile_of(blockIdx.x - n0, cdiv(SS.s[1].w, TW), cdiv(SS.s[1].h, TH), nz)
-                : tile_of(blockIdx.x, nx0, ny0, nz);
-}
-
-// 1 / (sum of the taps inside [0, n)) at position p in [0, n) for a window of
-// radius R (gaussianblur.hpp:63-65, 83-84).
-template <int R>
-__device__ __forceinline__ float inv_total(const Taps* __restrict__ T, int p, int n) {
-    const int lo = max(0, R - p), hi = min(2 * R, n - 1 - p + R);
-    return 1.0f / (T->cum[hi + 1] - T->cum[lo]);
-}
-
-// Column and row factors of an output region [x0, x0 + OW) x [y0, y0 + OH):
-// 0 outside the image.
-template <int R, int OW, int OH>
-__device__ __forceinline__ void edge_factors(float* colf, float* rowf, const Taps* __restrict__ T, int w, int h,
-                                             int x0, int y0) {
-    static_assert(OW <= 128 && OH <= 128, "factor threads");
-    const int t = threadIdx.x;
-    if (t < OW) {
-        const int gx = x0 + t;
-        colf[t] = (gx >= 0 && gx < w) ? inv_total<R>(T, gx, w) : 0.0f;
-    } else if (t >= 128 && t < 128 + OH) {
-        const int gy = y0 + t - 128;
-        rowf[t - 128] = (gy >= 0 && gy < h) ? inv_total<R>(T, gy, h) : 0.0f;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// point operations (src/butter/colors.hpp, separatefrequencies.hpp:3-50,
-// maskPsycho.hpp, combineMasks.hpp)
-// ---------------------------------------------------------------------------
-// sign(a) |a|^2.4 (colors.hpp:7-13) as 2^(2.4 log2|a|) on the hardware
-// exp2/log2 units: within a few ulp of powf, which costs an order of
-// magnitude more instructions. |a| is clamped to 1e-30, whose power
-// underflows to exactly 0, so 0 needs no branch.
-__device__ __forceinline__ float linearize(float a) {
-    const float m = fmaxf(fabsf(a), 1e-30f);
-    return copysignf(__builtin_amdgcn_exp2f(2.4f * __builtin_amdgcn_logf(m)), a);
-}
-
-// 19.245 ln(v + 9.971) - 23.160 with the logarithm on the hardware log2 unit
-// (1 ulp; its argument is above 11) and ln 2 folded into the factor
-__device__ __forceinline__ float opsin_gamma(float v) {
-    constexpr float kMul = (float)(19.245013259874995 * 0.69314718055994531);
-    return fmaf(kMul, __builtin_amdgcn_logf(v + 9.9710635769299145f), -23.16046239805755f);
-}
-
-__device__ __forceinline__ void opsin_absorbance(float a0, float a1, float a2, float& o0, float& o1, float& o2) {
-    o0 = fmaf(0.29956550340058319f, a0, fmaf(0.63373087833825936f, a1, fmaf(0.077705617820981968f, a2, 1.7557483643287353f)));
-    o1 = fmaf(0.22158691104574774f, a0, fmaf(0.69391388044116142f, a1, fmaf(0.0987313588422f, a2, 1.7557483643287353f)));
-    o2 = fmaf(0.02f, a0, fmaf(0.02f, a1, fmaf(0.20480129041026129f, a2, 12.226454707163354f)));
-}
-
-__device__ __forceinline__ float remove_range(float x, float w) { return x > w ? x - w : (x < -w ? x + w : 0.0f); }
-__device__ __forceinline__ float amplify_range(float x, float w) { return x > w ? x + w : (x < -w ? x - w : 2.0f * x); }
-__device__ __forceinline__ float maximum_clamp(float v, float maxval) {
-    const float mul = 0.688059627878f;
-    if (v >= maxval) return (v - maxval) * mul + maxval;
-    if (v < -maxval) return (v + maxval) * mul - maxval;
-    return v;
-}
-
-// mask input: amplitude of the high bands, compressed (maskinit + diffPrecompute)
-__device__ __forceinline__ float mask_input(float hfx, float uhfx, float hfy, float uhfy) {
-    const float xd = (uhfx + hfx) * 2.5f;
-    const float yd = uhfy * 0.4f + hfy * 0.4f;
-    // square roots of non-negative values on the hardware unit (1 ulp)
-    const float m = __builtin_amdgcn_sqrtf(xd * xd + yd * yd);
-    const float mul = 6.19424080439f, bias = mul * 12.61050594197f;
-    return __builtin_amdgcn_sqrtf(mul * fabsf(m) + bias) - __builtin_amdgcn_sqrtf(bias);
-}
-
-constexpr double kMaskNorm = 1.0 / (double)(0.79079917404f * 17.83f);
-
-__device__ __forceinline__ float mask_y(float d) {
-    // hardware reciprocal (1 ulp) of a denominator above 0.8
-    const float c = 2.5485944793f * __builtin_amdgcn_rcpf((0.451936922203f * d) + 0.829591754942f);
-    const float r = (float)((1.0 + (double)c) * kMaskNorm);
-    return r * r;
-}
-__device__ __forceinline__ float mask_dc_y(float d) {
-    const float c = 0.505054525019f * __builtin_amdgcn_rcpf((3.87449418804f * d) + 0.20025578522f);
-    const float r = (float)((1.0 + (double)c) * kMaskNorm);
-    return r * r;
-}
-
-// a * b rounded to FP32 on its own: never contracted into a following add
-// (where it would be kept exact), so that two values computed alike compare
-// equal however they are used
-__device__ __forceinline__ float mul_rounded(float a, float b) {
-#pragma clang fp contract(off)
-    return a * b;
-}
-
-// Insert v into the three smallest values m0 <= m1 <= m2 (StoreMin3,
-// maskPsycho.hpp:42-56), as a min/max network: the same three values for any
-// non-NaN v as the reference's branches, which the compiler would otherwise
-// lower to a private array written at a computed slot.
-__device__ __forceinline__ void store_min3(float v, float& m0, float& m1, float& m2) {
-    const float n2 = fminf(m2, fmaxf(m1, v));
-    const float n1 = fminf(m1, fmaxf(m0, v));
-    m0 = fminf(m0, v);
-    m1 = n1;
-    m2 = n2;
-}
 
 // ---------------------------------------------------------------------------
 // input: sample, linearise, 2x2 mean (Planed.hpp, colors.hpp:7-21,
@@ -303,7 +90,7 @@ __device__ __forceinline__ void yuv_rgb(const uint8_t* const* src, const int64_t
 
 template <int FMT>
 __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* __restrict__ pairs, Scale S0,
-                                                                Scale S1) {
+                                                                Scale S1, float scale) {
     const int pair = blockIdx.z;
     const int hx = blockIdx.x * 16 + (threadIdx.x & 15), hy = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (hx >= S1.w || hy >= S1.h) return;
@@ -333,8 +120,8 @@ __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* 
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const float a = linearize(v[0][c]), b = linearize(v[1][c]);
-            const float cc = linearize(v[2][c]), d = linearize(v[3][c]);
+            const float a = linearize(v[0][c]) * scale, b = linearize(v[1][c]) * scale;
+            const float cc = linearize(v[2][c]) * scale, d = linearize(v[3][c]) * scale;
             float* L = plane_of(S0, pair, P_LIN + im * 3 + c);
             L[(int64_t)y0 * S0.pitch + x0] = a;
             if (xo) L[(int64_t)y0 * S0.pitch + x1] = b;
@@ -357,7 +144,7 @@ __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* 
 // thread converts four 2 x 2 quads per image.
 template <bool WIDE>
 __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDesc* __restrict__ pairs, Scale S0,
-                                                                   Scale S1) {
+                                                                   Scale S1, float scale) {
     __shared__ float ch[2][kCh420][kCh420 + 1];
     const TileIdx ti = tile_of_block();
     const int pair = ti.z;
@@ -397,9 +184,9 @@ __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDes
                 const float yn = fmaf(yv[k], ymul, yadd);
                 const float R = fmaf(rcr, cr[k], yn);
                 const float B = fmaf(bcb, cb[k], yn);
-                lin[k][0] = linearize(R);
-                lin[k][1] = linearize((yn - kr * R - kb * B) * ikg);
-                lin[k][2] = linearize(B);
+                lin[k][0] = linearize(R) * scale;
+                lin[k][1] = linearize((yn - kr * R - kb * B) * ikg) * scale;
+                lin[k][2] = linearize(B) * scale;
             }
             // each row's two pixels as one 8-byte store (xa is even and rows are
             // padded to 64 floats: with no second column, at an odd width, the
@@ -423,14 +210,14 @@ __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDes
 }
 
 template <int FMT>
-void launch_input(dim3 g, hipStream_t st, const PairDesc* pairs, const Scale& S0, const Scale& S1) {
-    butter_input_kernel<FMT><<<g, dim3(kThreads), 0, st>>>(pairs, S0, S1);
+void launch_input(dim3 g, hipStream_t st, const PairDesc* pairs, const Scale& S0, const Scale& S1, float scale) {
+    butter_input_kernel<FMT><<<g, dim3(kThreads), 0, st>>>(pairs, S0, S1, scale);
 }
 
 template <int... F>
 void launch_input_fmt(int fmt, dim3 g, hipStream_t st, const PairDesc* pairs, const Scale& S0, const Scale& S1,
-                      std::integer_sequence<int, F...>) {
-    ((fmt == F ? launch_input<F>(g, st, pairs, S0, S1) : void()), ...);
+                      float scale, std::integer_sequence<int, F...>) {
+    ((fmt == F ? launch_input<F>(g, st, pairs, S0, S1, scale) : void()), ...);
 }
 
 // ---------------------------------------------------------------------------
@@ -722,18 +509,9 @@ __global__ __launch_bounds__(kThreads) void butter_opsin_kernel(Scales SS, int n
     for (int i = 0; i < kRun; i++) {
         float b0, b1, b2;
         opsin_absorbance(bl[0][i] * intensity, bl[1][i] * intensity, bl[2][i] * intensity, b0, b1, b2);
-        b0 = fmaxf(fmaxf(b0, 1.7557483643287353f), 1e-4f);
-        b1 = fmaxf(fmaxf(b1, 1.7557483643287353f), 1e-4f);
-        b2 = fmaxf(fmaxf(b2, 12.226454707163354f), 1e-4f);
-        // b >= 1.75: the hardware reciprocal (1 ulp) for the reference's division
-        const float s0 = fmaxf(opsin_gamma(b0) * __builtin_amdgcn_rcpf(b0), 1e-4f);
-        const float s1 = fmaxf(opsin_gamma(b1) * __builtin_amdgcn_rcpf(b1), 1e-4f);
-        const float s2 = fmaxf(opsin_gamma(b2) * __builtin_amdgcn_rcpf(b2), 1e-4f);
         float o0, o1, o2;
         opsin_absorbance(ctr[0][i] * intensity, ctr[1][i] * intensity, ctr[2][i] * intensity, o0, o1, o2);
-        o0 = fmaxf(o0 * s0, 1.7557483643287353f);
-        o1 = fmaxf(o1 * s1, 1.7557483643287353f);
-        o2 = fmaxf(o2 * s2, 12.226454707163354f);
+        opsin_respond(b0, b1, b2, o0, o1, o2);
         x[i] = o0 - o1;
         y[i] = o0 + o1;
         z[i] = o2;
@@ -958,51 +736,6 @@ __device__ __forceinline__ void malta_block(const float* __restrict__ win_origin
     }
 }
 
-// One Malta term: the scaled differences of the two planes.
-struct MaltaTerm {
-    float n2gt, n2lt, norm1;
-};
-
-// The two weights share one hardware reciprocal (1 ulp) of
-// norm1 + |a|/2 + |b|/2; the reference divides twice, and the results differ
-// by rounding only.
-//
-// The impact term is formed without branches: with b mirrored to bm = -b when
-// a < 0, the reference's two cases (maltaDiff.hpp:553-572) are the one case
-// a >= 0, and too_small - bm, bm - too_big are exactly its b + too_small,
-// -b - too_big (negation is exact), so the value is bit-identical.
-__device__ __forceinline__ float malta_scaled_diff(float a, float b, const MaltaTerm& M) {
-    const float fabs0 = fabsf(a);
-    const float absval = 0.5f * fabs0 + 0.5f * fabsf(b);
-    const float diff = a - b;
-    const float inv = __builtin_amdgcn_rcpf(M.norm1 + absval);
-    const float v = (M.n2gt * inv) * diff;
-    const float scaler2 = M.n2lt * inv;
-    const float too_small = 0.55f * fabs0, too_big = 1.05f * fabs0;
-    const float bm = a < 0.0f ? -b : b;
-    float impact = bm < too_small ? too_small - bm : (bm > too_big ? bm - too_big : 0.0f);
-    impact *= scaler2;
-    return diff < 0.0f ? v - impact : v + impact;
-}
-
-struct DiffParams {
-    MaltaTerm malta[6];  // uhf Y, uhf X, hf Y, hf X, mf Y, mf X
-    float asym_gt[2], asym_lt[2];
-};
-
-// asymmetric L2 term (simplerdiff.hpp:60-90), its cases folded as in
-// malta_scaled_diff (bit-identical)
-__device__ __forceinline__ float l2_asym(float a, float b, float wgt, float wlt) {
-    const float diff = a - b;
-    float r = wgt * diff * diff;
-    const float fabs0 = fabsf(a);
-    // 0.4 * |a| is a double product rounded to float in simplerdiff.hpp:69
-    const float too_small = (float)(0.4 * (double)fabs0), too_big = fabs0;
-    const float bm = a < 0.0f ? -b : b;
-    const float v = bm < too_small ? too_small - bm : (bm > too_big ? bm - too_big : 0.0f);
-    return r + wlt * v * v;
-}
-
 __global__ __launch_bounds__(kThreads) void butter_diff_kernel(Scales SS, int nz, DiffParams D) {
     __shared__ float dt[kDSH * kDSW];
     Scale S;
@@ -1087,6 +820,56 @@ __global__ __launch_bounds__(kThreads) void butter_diff_kernel(Scales SS, int nz
         at(plane_u(S, pair, P_DCS), g) = dc;
         at(plane_u(S, pair, P_M0), g) = mask_input(hf[0][0], uhf[0][0], hf[0][1], uhf[0][1]);
         at(plane_u(S, pair, P_M1), g) = mask_input(hf[1][0], uhf[1][0], hf[1][1], uhf[1][1]);
+    }
+}
+
+// The Malta terms of scaled differences that the matrix-core stages have
+// formed (planes Q_SD), added to the L2 terms in P_ACS.
+__global__ __launch_bounds__(kThreads) void butter_malta_kernel(Scales SS, int nz) {
+    __shared__ float dt[kDSH * kDSW];
+    Scale S;
+    const TileIdx ti = tile_of_scales<kDW, kDH>(SS, nz, S);
+    const int pair = ti.z;
+    const int ox0 = ti.x * kDW, oy0 = ti.y * kDH;
+    const int tx = threadIdx.x & (kDW - 1), ty = threadIdx.x / kDW;
+    const int w = S.w, h = S.h;
+    float ac[kDRows];
+#pragma unroll
+    for (int j = 0; j < kDRows; j++) ac[j] = 0.0f;
+#pragma unroll 1
+    for (int t = 0; t < 6; t++) {
+        const float* a = plane_u(S, pair, Q_SD + t);
+        constexpr int NE = (kDSW * kDSH + kThreads - 1) / kThreads;
+        float va[NE];
+#pragma unroll
+        for (int k = 0; k < NE; k++) {
+            const int i = threadIdx.x + k * kThreads;
+            const int r = i / kDSW, c = i - r * kDSW;
+            const int gx = ox0 - kDHalo + c, gy = oy0 - kDHalo + min(r, kDSH - 1);
+            const bool ok = i < kDSW * kDSH && gx >= 0 && gx < w && gy >= 0 && gy < h;
+            const float x = at(a, min(max(gy, 0), h - 1) * S.pitch + min(max(gx, 0), w - 1));
+            va[k] = ok ? x : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NE; k++) {
+            const int i = threadIdx.x + k * kThreads;
+            if (i < kDSW * kDSH) dt[i] = va[k];
+        }
+        __syncthreads();
+        const float* origin = dt + (kDRows * ty) * kDSW + tx;
+        if (t < 2)
+            malta_block<true>(origin, ac);
+        else
+            malta_block<false>(origin, ac);
+    }
+    const int gx = ox0 + tx;
+    if (gx >= w) return;
+    float* acs = plane_u(S, pair, P_ACS);
+#pragma unroll
+    for (int j = 0; j < kDRows; j++) {
+        const int gy = oy0 + kDRows * ty + j;
+        if (gy < h) at(acs, gy * S.pitch + gx) += ac[j];
     }
 }
 
@@ -1266,9 +1049,12 @@ __global__ __launch_bounds__(kThreads) void butter_mask_kernel(Scale S, const Ta
     }
 }
 
-// norms of each pair from its tile partials (diffnorms.hpp:85-127)
+// norms of each pair from its tile partials (diffnorms.hpp:85-127), and whether
+// it has to be scored again by the general kernels
 __global__ __launch_bounds__(kThreads) void butter_norm_kernel(const double* __restrict__ partials, int tiles,
-                                                               int qnorm, int64_t npix, double* __restrict__ norms) {
+                                                               int qnorm, int64_t npix,
+                                                               const PairDesc* __restrict__ pairs,
+                                                               double* __restrict__ norms) {
     __shared__ double red[3][kThreads / 64];
     const int pair = blockIdx.x;
     const double* p = partials + (int64_t)pair * tiles * 3;
@@ -1295,9 +1081,10 @@ __global__ __launch_bounds__(kThreads) void butter_norm_kernel(const double* __r
             sb += red[1][k];
             sm = fmax(sm, red[2][k]);
         }
-        norms[3 * pair + 0] = pow(sa / (double)npix, 1.0 / (double)qnorm);
-        norms[3 * pair + 1] = pow(sb / (double)npix, 1.0 / 3.0);
-        norms[3 * pair + 2] = sm;
+        norms[4 * pair + 0] = pow(sa / (double)npix, 1.0 / (double)qnorm);
+        norms[4 * pair + 1] = pow(sb / (double)npix, 1.0 / 3.0);
+        norms[4 * pair + 2] = sm;
+        norms[4 * pair + 3] = (double)pairs[pair].general;
     }
 }
 
@@ -1356,8 +1143,8 @@ Engine::Engine(int width, int height, int capacity, int qnorm, float intensity, 
         HIP_OR_THROW(hipMalloc(&arena_, arena), E_OutOfVRAM);
         mask_tiles_ = cdiv(w_, kMT) * cdiv(h_, kMT);
         HIP_OR_THROW(hipMalloc(&partials_d_, sizeof(double) * 3 * mask_tiles_ * cap_), E_OutOfVRAM);
-        HIP_OR_THROW(hipMalloc(&norms_d_, sizeof(double) * 3 * cap_), E_OutOfVRAM);
-        HIP_OR_THROW(hipHostMalloc(&norms_h_, sizeof(double) * 3 * cap_), E_OutOfRAM);
+        HIP_OR_THROW(hipMalloc(&norms_d_, sizeof(double) * 4 * cap_), E_OutOfVRAM);
+        HIP_OR_THROW(hipHostMalloc(&norms_h_, sizeof(double) * 4 * cap_), E_OutOfRAM);
         HIP_OR_THROW(hipMalloc(&desc_d_, sizeof(PairDesc) * cap_), E_OutOfVRAM);
         HIP_OR_THROW(hipHostMalloc(&desc_h_, sizeof(PairDesc) * cap_), E_OutOfRAM);
         HIP_OR_THROW(hipMalloc(&taps_d_, sizeof(Taps) * kSigmaCount), E_OutOfVRAM);
@@ -1376,6 +1163,10 @@ Engine::Engine(int width, int height, int capacity, int qnorm, float intensity, 
             th[i].cum[2 * R + 1] = (float)(run / tot);
         }
         HIP_OR_THROW(hipMemcpy(taps_d_, th, sizeof(th), hipMemcpyHostToDevice), E_BadDeviceArgument);
+        auto strip = std::make_unique<StripTables>();
+        fill_strip_tables(*strip);
+        HIP_OR_THROW(hipMalloc(&strip_d_, sizeof(StripTables)), E_OutOfVRAM);
+        HIP_OR_THROW(hipMemcpy(strip_d_, strip.get(), sizeof(StripTables), hipMemcpyHostToDevice), E_BadDeviceArgument);
         for (auto& e : ev_) HIP_OR_THROW(hipEventCreate(&e), E_BadDeviceArgument);
     } catch (...) {
         release();
@@ -1396,10 +1187,11 @@ void Engine::release() {
     if (desc_d_) (void)hipFree(desc_d_), desc_d_ = nullptr;
     if (desc_h_) (void)hipHostFree(desc_h_), desc_h_ = nullptr;
     if (taps_d_) (void)hipFree(taps_d_), taps_d_ = nullptr;
+    if (strip_d_) (void)hipFree(strip_d_), strip_d_ = nullptr;
     if (stream_) (void)hipStreamDestroy(stream_), stream_ = nullptr;
 }
 
-void Engine::submit(int fmt, const PairDesc* pairs, int n) {
+void Engine::run(int fmt, const PairDesc* pairs, int n, double* norms) {
     if (n <= 0 || n > cap_ || !pairs) VSHIP_THROW(E_BadPointer);
     if (fmt < 0 || fmt >= IN_NUM_FORMATS) VSHIP_THROW(E_BadPointer);
     // bytes per sample and plane widths of the format: every row the kernel
@@ -1428,33 +1220,55 @@ void Engine::submit(int fmt, const PairDesc* pairs, int n) {
         }
     }
     HIP_OR_THROW(hipSetDevice(device_), E_BadDeviceArgument);
-    // the previous batch may still read the pinned descriptors
-    HIP_OR_THROW(hipStreamSynchronize(stream_), E_BadDeviceArgument);
     // 4:2:0 batches whose pairs all have left-located chroma take the staged
     // input kernel
     staged420_ = fmt == IN_YUV420_U8 || fmt == IN_YUV420_U16;
     for (int i = 0; i < n && staged420_; i++) staged420_ = pairs[i].cloc == CLOC_LEFT;
+    last_fmt_ = fmt;
+    last_n_ = n;
+    score(fmt, pairs, n, false);
+    // a pair with values beyond the range of the matrix-core stages is scored
+    // by the general kernels
+    std::vector<PairDesc> again;
+    std::vector<int> which;
+    for (int i = 0; i < n; i++) {
+        if (norms) std::memcpy(norms + 3 * i, norms_h_ + 4 * i, sizeof(double) * 3);
+        if (norms_h_[4 * i + 3] != 0.0) {
+            again.push_back(pairs[i]);
+            which.push_back(i);
+        }
+    }
+    if (again.empty()) return;
+    score(fmt, again.data(), (int)again.size(), true);
+    for (size_t k = 0; norms && k < which.size(); k++)
+        std::memcpy(norms + 3 * which[k], norms_h_ + 4 * k, sizeof(double) * 3);
+}
+
+void Engine::score(int fmt, const PairDesc* pairs, int n, bool general) {
+    // a batch that ended in an error may still read the pinned descriptors
+    if (in_flight_) HIP_OR_THROW(hipStreamSynchronize(stream_), E_BadDeviceArgument);
+    in_flight_ = true;
     std::memcpy(desc_h_, pairs, sizeof(PairDesc) * n);
+    for (int i = 0; i < n; i++) desc_h_[i].general = 0;
     HIP_OR_THROW(hipMemcpyAsync(desc_d_, desc_h_, sizeof(PairDesc) * n, hipMemcpyHostToDevice, stream_),
                  E_BadDeviceArgument);
-    launch(fmt, n);
-    last_fmt_ = fmt;
-    HIP_OR_THROW(hipMemcpyAsync(norms_h_, norms_d_, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, stream_),
+    launch(fmt, n, general);
+    HIP_OR_THROW(hipMemcpyAsync(norms_h_, norms_d_, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, stream_),
                  E_BadDeviceArgument);
-    last_n_ = n;
-}
-
-void Engine::run(int fmt, const PairDesc* pairs, int n, double* norms) {
-    submit(fmt, pairs, n);
     HIP_OR_THROW(hipStreamSynchronize(stream_), E_BadDeviceArgument);
-    if (norms) std::memcpy(norms, norms_h_, sizeof(double) * 3 * n);
+    in_flight_ = false;
 }
 
-void Engine::launch(int fmt, int n) {
+void Engine::launch(int fmt, int n, bool general) {
     const Scale S0{arena_, w_, h_, row_pitch(w_), plane0_, (int64_t)P_COUNT * plane0_};
     const Scale S1{arena_ + (int64_t)cap_ * P_COUNT * plane0_, w2_, h2_, row_pitch(w2_), plane1_,
                    (int64_t)P_COUNT * plane1_};
-    const DiffParams D = diff_params();
+    StripArgs A;
+    A.pairs = desc_d_;
+    A.intensity = intensity_ / kLinScale;
+    A.diff = diff_params();
+    const float lin = general ? 1.0f : kLinScale;
+    const int th = strip_height(w_, h_, w2_, h2_, n);
     const bool prof = profile_;
     auto mark = [&](int st) {
         if (prof) (void)hipEventRecord(ev_[st], stream_);
@@ -1464,12 +1278,12 @@ void Engine::launch(int fmt, int n) {
         if (staged420_) {
             const dim3 g4(cdiv(w_, 64), cdiv(h_, 64), n);
             if (fmt == IN_YUV420_U16)
-                butter_input420_kernel<true><<<g4, dim3(kThreads), 0, stream_>>>(desc_d_, S0, S1);
+                butter_input420_kernel<true><<<g4, dim3(kThreads), 0, stream_>>>(desc_d_, S0, S1, lin);
             else
-                butter_input420_kernel<false><<<g4, dim3(kThreads), 0, stream_>>>(desc_d_, S0, S1);
+                butter_input420_kernel<false><<<g4, dim3(kThreads), 0, stream_>>>(desc_d_, S0, S1, lin);
             return;
         }
-        launch_input_fmt(fmt, gi, stream_, desc_d_, S0, S1, std::make_integer_sequence<int, IN_NUM_FORMATS>{});
+        launch_input_fmt(fmt, gi, stream_, desc_d_, S0, S1, lin, std::make_integer_sequence<int, IN_NUM_FORMATS>{});
     };
     const Scales SS{{S0, S1}};
     // workgroups of a two-scale launch with tiles of tw x th and nz plane sets
@@ -1496,19 +1310,33 @@ void Engine::launch(int fmt, int n) {
         switch (st) {
             case ST_INPUT: input(); break;
             case ST_OPSIN:
-                butter_opsin_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_, intensity_);
+            case ST_LOW:
+            case ST_MID:
+            case ST_HIGH: {
+                if (!general) {
+                    launch_strip_stage(st, SS, n, th, strip_d_, A, stream_);
+                    break;
+                }
+                const dim3 g = grid2(kTW, kTH, 2 * n);
+                if (st == ST_OPSIN) butter_opsin_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_, intensity_);
+                if (st == ST_LOW) butter_low_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_);
+                if (st == ST_MID) butter_mid_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_);
+                if (st == ST_HIGH) butter_high_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_);
                 break;
-            case ST_LOW: butter_low_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_); break;
-            case ST_MID: butter_mid_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_); break;
-            case ST_HIGH: butter_high_kernel<<<grid2(kTW, kTH, 2 * n), blk, 0, stream_>>>(SS, 2 * n, taps_d_); break;
-            case ST_DIFF: butter_diff_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n, D); break;
+            }
+            case ST_DIFF:
+                if (general)
+                    butter_diff_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n, A.diff);
+                else
+                    butter_malta_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n);
+                break;
             case ST_MASK:
                 mask(S1, false);  // the full scale blends its map with this one's
                 mask(S0, true);
                 break;
             default:
                 butter_norm_kernel<<<dim3(n), blk, 0, stream_>>>(partials_d_, mask_tiles_, q_, (int64_t)w_ * h_,
-                                                                 norms_d_);
+                                                                 desc_d_, norms_d_);
         }
     };
     for (int st = 0; st < ST_COUNT; st++) {

@@ -30,6 +30,7 @@ struct PairDesc {
     int32_t bits;
     int32_t cloc;
     float kr, kb;
+    int32_t general;  // set by the kernels: a value beyond the range of the matrix-core stages
 };
 
 // Kernel groups, for per-kernel timing.
@@ -45,6 +46,8 @@ enum Stage : int {
     ST_COUNT
 };
 
+struct StripTables;
+
 class Engine {
 public:
     // Throws VshipErr (E_OutOfVRAM, E_BadDeviceArgument) on failure.
@@ -58,10 +61,6 @@ public:
     // norms[3 * i .. 3 * i + 2] = Q-norm, 3-norm, max of pair i.
     // Synchronous; the work runs on stream().
     void run(int fmt, const PairDesc* pairs, int n, double* norms);
-
-    // Enqueue only; the norms land in norms_host() after a stream sync.
-    void submit(int fmt, const PairDesc* pairs, int n);
-    const double* norms_host() const { return norms_h_; }
 
     hipStream_t stream() const { return stream_; }
     int width() const { return w_; }
@@ -79,7 +78,9 @@ public:
     static uint64_t pair_bytes(int width, int height);
 
 private:
-    void launch(int fmt, int n);
+    // Uploads the descriptors, runs every stage and waits for the norms.
+    void score(int fmt, const PairDesc* pairs, int n, bool general);
+    void launch(int fmt, int n, bool general);
     void release();
 
     int w_, h_, w2_, h2_, cap_, q_;
@@ -90,10 +91,12 @@ private:
     int last_n_ = 0;
     int last_fmt_ = IN_RGB_F32;
     bool staged420_ = false;
+    bool in_flight_ = false;
     hipStream_t stream_ = nullptr;
     float* arena_ = nullptr;
     int64_t plane0_ = 0, plane1_ = 0;
     Taps* taps_d_ = nullptr;
+    StripTables* strip_d_ = nullptr;
     PairDesc* desc_d_ = nullptr;
     PairDesc* desc_h_ = nullptr;
     double* partials_d_ = nullptr;
