@@ -189,22 +189,32 @@ __device__ __forceinline__ void opsin_respond(float b0, float b1, float b2, floa
 }
 
 __device__ __forceinline__ float remove_range(float x, float w) { return x > w ? x - w : (x < -w ? x + w : 0.0f); }
-__device__ __forceinline__ float amplify_range(float x, float w) { return x > w ? x + w : (x < -w ? x - w : 2.0f * x); }
+// the reference's three cases x > w, x < -w and between as one sum with x
+// clamped to [-w, w]: the same values, without branches
+__device__ __forceinline__ float amplify_range(float x, float w) { return x + fminf(fmaxf(x, -w), w); }
 __device__ __forceinline__ float maximum_clamp(float v, float maxval) {
-    const float mul = 0.688059627878f;
-    if (v >= maxval) return (v - maxval) * mul + maxval;
-    if (v < -maxval) return (v + maxval) * mul - maxval;
-    return v;
+    const float c = fminf(fmaxf(v, -maxval), maxval);
+    return (v - c) * 0.688059627878f + c;
+}
+
+// a * b rounded to FP32 on its own: never contracted into a following add
+// (where it would be kept exact), so that two values computed alike compare
+// equal however they are used
+__device__ __forceinline__ float mul_rounded(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
 }
 
 // mask input: amplitude of the high bands, compressed (maskinit + diffPrecompute)
 __device__ __forceinline__ float mask_input(float hfx, float uhfx, float hfy, float uhfy) {
+    // the sums of products are written as the fmas they become, so that both
+    // images' are rounded alike wherever this is inlined
     const float xd = (uhfx + hfx) * 2.5f;
-    const float yd = uhfy * 0.4f + hfy * 0.4f;
+    const float yd = fmaf(uhfy, 0.4f, mul_rounded(hfy, 0.4f));
     // square roots of non-negative values on the hardware unit (1 ulp)
-    const float m = __builtin_amdgcn_sqrtf(xd * xd + yd * yd);
+    const float m = __builtin_amdgcn_sqrtf(fmaf(xd, xd, mul_rounded(yd, yd)));
     const float mul = 6.19424080439f, bias = mul * 12.61050594197f;
-    return __builtin_amdgcn_sqrtf(mul * fabsf(m) + bias) - __builtin_amdgcn_sqrtf(bias);
+    return __builtin_amdgcn_sqrtf(fmaf(mul, fabsf(m), bias)) - __builtin_amdgcn_sqrtf(bias);
 }
 
 constexpr double kMaskNorm = 1.0 / (double)(0.79079917404f * 17.83f);
@@ -219,14 +229,6 @@ __device__ __forceinline__ float mask_dc_y(float d) {
     const float c = 0.505054525019f * __builtin_amdgcn_rcpf((3.87449418804f * d) + 0.20025578522f);
     const float r = (float)((1.0 + (double)c) * kMaskNorm);
     return r * r;
-}
-
-// a * b rounded to FP32 on its own: never contracted into a following add
-// (where it would be kept exact), so that two values computed alike compare
-// equal however they are used
-__device__ __forceinline__ float mul_rounded(float a, float b) {
-#pragma clang fp contract(off)
-    return a * b;
 }
 
 // Insert v into the three smallest values m0 <= m1 <= m2 (StoreMin3,

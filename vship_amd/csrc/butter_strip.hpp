@@ -25,7 +25,7 @@ enum : int {
 };
 static_assert(Q_T == Q_DB + 1 && Q_HFR == Q_T + 5 && Q_COUNT <= P_ACS, "plane layout");
 
-constexpr int kStripOps = 6;
+constexpr int kStripOps = 4;
 struct StripTables {
     uint32_t op[kSigmaCount][kStripOps][2][64][4];  // tap operands: [h, l][lane][8 fp16]
     Taps taps[kSigmaCount];                         // the taps as the operands represent them
