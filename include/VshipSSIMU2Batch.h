@@ -140,7 +140,8 @@ typedef struct {
     float prep_ms;      /* convert + pyramid + XYB kernel */
     float map_ms;       /* blur + SSIM/edge maps, both precision classes */
     float map_fp32_ms;  /* map kernel of the segments with FP32 moment accumulation */
-    float map_fp64_ms;  /* map kernel of the small segments (FP64 moment accumulation) */
+    float map_fp64_ms;  /* map kernel of the small segments (FP64 moment accumulation); about 0 where they
+                           ride along with the matrix-core kernel (an eager launch of one workgroup per tile) */
     float finalize_ms;  /* FP64 norms + score kernel */
     float total_ms;     /* whole batch, first copy to last copy */
     int npairs;

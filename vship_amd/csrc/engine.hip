@@ -117,6 +117,8 @@ int map_tiles(int w, int h, int th) {
     return n;
 }
 
+int max_map_tiles(int w, int h) { return map_tiles(w, h, 32) + kSmallTilesMax; }
+
 uint64_t map_algorithmic_bytes(int w, int h, bool fp16) {
     uint64_t t = 0;
     int ww = w, hh = h;
@@ -163,7 +165,6 @@ Engine::Engine(const EngineOptions& opt) : opt_(opt) {
         if (max_map_tiles_ <= 0) VSHIP_THROW(E_OutOfVRAM);
         HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&partials_d_), sizeof(double) * kFeat * max_map_tiles_),
                      E_OutOfVRAM);
-        HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&out_d_), out_bytes), E_OutOfVRAM);
     } catch (...) {
         release();
         throw;
@@ -199,13 +200,11 @@ void Engine::release() {
         in_d_[k] = nullptr;
         in_cap_[k] = 0;
     }
-    if (out_d_) (void)hipFree(out_d_);
     if (partials_d_) (void)hipFree(partials_d_);
     if (arena_d_) (void)hipFree(arena_d_);
     if (desc_d_) (void)hipFree(desc_d_);
     if (copy_) (void)hipStreamDestroy(copy_);
     if (stream_) (void)hipStreamDestroy(stream_);
-    out_d_ = nullptr;
     partials_d_ = nullptr;
     arena_d_ = nullptr;
     desc_d_ = nullptr;
@@ -308,7 +307,7 @@ PlanInfo plan_batch(const PairInput* in, int n, int max_pairs, bool fp16, int ma
                 if ((mfma && cls == 0 && float_in) != exact) continue;
                 if (((int64_t)sw * sh < (mfma ? kSmallSegmentMx : kSmallSegment) ? 1 : 0) != cls) continue;
                 if ((fp16 && s < kHalfScales) != half) continue;
-                const int th = cls ? kSmallTH : map_th;
+                const int th = cls ? (mfma ? kMapSmall : kSmallTH) : map_th;
                 const int tw = map_tile_w(th), tht = map_tile_h(th);
                 const int64_t cnt = (int64_t)((sw + tw - 1) / tw) * ((sh + tht - 1) / tht);
                 const int seg = i * kScales + s;
@@ -359,15 +358,25 @@ void launch_batch(const DescView& d, const PlanInfo& P, const LaunchShape& S, vo
     };
     const int g_prep = grid_for(P.ntiles_prep, fixed);
     const int g_fin = grid_for(P.npairs, std::min(S.max_pairs, fixed));
-    HIP_OR_THROW(launch_prep(S.fp16, false, g_prep, d.pairs, d.prep_start, d.hdr, arena, st), E_BadDeviceCode);
-    // pairs on the generic chroma path have their own prep kernel; a captured
-    // graph always holds it (it returns at once when the batch has none)
+    // pairs on the generic chroma path have their own prep kernel, and a batch
+    // of only such pairs no other; a captured graph always holds both (each
+    // returns at once when the batch has none of its pairs)
+    if (graph || P.nprep_generic < P.npairs)
+        HIP_OR_THROW(launch_prep(S.fp16, false, g_prep, d.pairs, d.prep_start, d.hdr, arena, st), E_BadDeviceCode);
     if (graph || P.nprep_generic > 0)
         HIP_OR_THROW(launch_prep(S.fp16, true, g_prep, d.pairs, d.prep_start, d.hdr, arena, st), E_BadDeviceCode);
     if (ev) HIP_OR_THROW(hipEventRecord(ev[0], st), E_BadDeviceCode);
     // one launch per map group; FP16-plane groups exist only with FP16 storage,
     // and an eager launch is skipped when its group is empty
     const bool mfma = S.map_th == kMapMfma;
+    // An eager launch of the matrix-core kernel brings the FP64 tiles of its
+    // plane storage along, a workgroup per tile and channel ahead of its own:
+    // by themselves these few workgroups, whose time is latency, held the GPU
+    // for 14 us of a 1920 x 1080 pair's 116.
+    const bool merged = mfma && !graph && S.persistent_grid == 0;
+    int small[2] = {};  // FP64 workgroups still to be launched, by plane storage
+    if (merged)
+        for (int half = 0; half < 2; half++) small[half] = 3 * P.ntiles_grp[map_group(1, half)];
     for (int cls = 0; cls < 2; cls++) {
         // on the matrix cores, class 0 also has the exact-split groups of float-input pairs
         const int nexact = (cls == 0 && mfma) ? 2 : 1;
@@ -375,25 +384,34 @@ void launch_batch(const DescView& d, const PlanInfo& P, const LaunchShape& S, vo
             for (int half = 0; half < 2; half++) {
                 const int g = map_group(cls, half, exact);
                 if (half && !S.fp16) continue;
-                if (!graph && P.ntiles_grp[g] == 0) continue;
+                const int nsmall = cls == 0 && (P.ntiles_grp[g] > 0 || exact == 1) ? small[half] : 0;
+                if (!graph && P.ntiles_grp[g] == 0 && nsmall == 0) continue;
+                if (merged && cls == 1) continue;
                 // an eager launch of few tiles gives each channel of a tile its
                 // own workgroup (the same partials): fewer than two tiles per
                 // workgroup slot on the matrix-core kernel (4 per CU), and for
                 // the vector kernels (as few as 1 workgroup per CU in the FP64
                 // class) when the split workgroups fit in two rounds, as for
                 // one pair per call
-                const bool small = (cls == 0 && mfma) ? P.ntiles_grp[g] < 8 * S.num_cus
-                                                      : 3 * P.ntiles_grp[g] <= 2 * S.num_cus;
-                const int csplit = (!graph && S.persistent_grid == 0 && small) ? 3 : 1;
-                const int grid = grid_for(P.ntiles_grp[g] * csplit, cls == 0 ? fixed : std::max(1, fixed / 4));
-                if (cls == 0 && mfma)
-                    HIP_OR_THROW(launch_map_mx(half, exact, grid, d.pairs, d.order_seg, d.order_start, d.hdr, arena,
-                                               partials, csplit, st),
+                const bool few = (cls == 0 && mfma) ? P.ntiles_grp[g] < 8 * S.num_cus
+                                                    : 3 * P.ntiles_grp[g] <= 2 * S.num_cus;
+                const int csplit = (!graph && S.persistent_grid == 0 && few) ? 3 : 1;
+                if (cls == 0 && mfma) {
+                    const int grid = P.ntiles_grp[g] > 0 || graph ? grid_for(P.ntiles_grp[g] * csplit, fixed) : 0;
+                    HIP_OR_THROW(launch_map_mx(half, exact, grid, nsmall, d.pairs, d.order_seg, d.order_start, d.hdr,
+                                               arena, partials, csplit, st),
                                  E_BadDeviceCode);
-                else
+                    small[half] -= nsmall;
+                } else if (mfma) {
+                    HIP_OR_THROW(launch_map_small(half, grid_for(3 * P.ntiles_grp[g], fixed), d.pairs, d.order_seg,
+                                                  d.order_start, d.hdr, arena, partials, st),
+                                 E_BadDeviceCode);
+                } else {
+                    const int grid = grid_for(P.ntiles_grp[g] * csplit, cls == 0 ? fixed : std::max(1, fixed / 4));
                     HIP_OR_THROW(launch_map(half, cls, cls ? kSmallTH : S.map_th, grid, d.pairs, d.order_seg,
                                             d.order_start, d.hdr, arena, partials, taps, csplit, st),
                                  E_BadDeviceCode);
+                }
             }
         if (ev) HIP_OR_THROW(hipEventRecord(ev[1 + cls], st), E_BadDeviceCode);
     }
@@ -416,16 +434,10 @@ void Engine::enqueue_body(int k) {
     HIP_OR_THROW(hipMemcpyAsync(desc_d_, desc_h_[k], desc_.bytes, hipMemcpyHostToDevice, stream_),
                  E_BadDeviceCode);
     if (prof) HIP_OR_THROW(hipEventRecord(ev[1], stream_), E_BadDeviceCode);
-    double* scores_d = out_d_;
-    double* feats_d = out_d_ + opt_.max_pairs;
-    launch_batch(desc_view(desc_d_, desc_), plan_, S, arena_d_, partials_d_, scores_d, feats_d, taps_, stream_,
-                 prof ? ev + 2 : nullptr);
-    // scores [0, max_pairs) and features [max_pairs, ...) are one block on
-    // both sides: one copy brings back the scores and the batch's features
-    const int np = opt_.use_graph ? opt_.max_pairs : plan_.npairs;
-    HIP_OR_THROW(hipMemcpyAsync(out_h_[k], scores_d, sizeof(double) * (opt_.max_pairs + 108 * (size_t)np),
-                                hipMemcpyDeviceToHost, stream_),
-                 E_BadDeviceCode);
+    // the finalize kernel writes scores and features to the slot's page-locked
+    // result buffer itself: a copy behind it costs more than their bytes
+    launch_batch(desc_view(desc_d_, desc_), plan_, S, arena_d_, partials_d_, out_h_[k], out_h_[k] + opt_.max_pairs,
+                 taps_, stream_, prof ? ev + 2 : nullptr);
     if (prof) HIP_OR_THROW(hipEventRecord(ev[6], stream_), E_BadDeviceCode);
 }
 

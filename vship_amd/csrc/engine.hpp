@@ -104,6 +104,7 @@ PairLayout pair_layout(int w, int h, bool fp16);
 int64_t pair_bytes(int w, int h, bool fp16);  // arena bytes of both images
 int prep_tiles(int w, int h);
 int map_tiles(int w, int h, int th);
+int max_map_tiles(int w, int h);  // of a pair, whatever the tile shape
 uint64_t map_algorithmic_bytes(int w, int h, bool fp16);
 uint64_t prep_algorithmic_bytes(const PairInput& p, bool fp16);
 
@@ -215,8 +216,7 @@ private:
     int64_t arena_bytes_ = 0;
     double* partials_d_ = nullptr;
     int64_t max_map_tiles_ = 0;
-    double* out_d_ = nullptr;   // scores [max_pairs] then features [max_pairs*108]
-    double* out_h_[kDepth] = {};  // pinned, same layout
+    double* out_h_[kDepth] = {};  // pinned, written by the kernels: scores [max_pairs] then features [max_pairs*108]
     hipEvent_t ev_[kDepth][7] = {};
     hipEvent_t done_[kDepth] = {};
     hipGraph_t graph_[kDepth] = {};

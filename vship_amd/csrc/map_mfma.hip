@@ -50,6 +50,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernel_util.hpp"
+#include "map_small.hpp"
 #include "ssimu2_dev.hpp"
 #include "ssimu2_kernels.hpp"
 
@@ -602,16 +603,28 @@ __device__ __forceinline__ void mx_tile(MxLds<SP::kParts>& L, const TileGeo& T, 
 // (work item w: tile w / 3, channel w % 3), for batches with too few tiles to
 // fill the GPU. A channel's sums do not depend on the others, so both give
 // the same partials bit for bit.
+//
+// The first nsmall workgroups take the FP64 tiles of this plane storage, one
+// channel of one tile each.
 template <typename ST, typename SP>
 __global__ __launch_bounds__(256, SP::kParts == 2 ? 4 : 2) void map_mx_kernel(const PairDev* __restrict__ pairs,
                                                         const int32_t* __restrict__ order_seg,
                                                         const int32_t* __restrict__ order_start,
                                                         const BatchHdr* __restrict__ hdr,
                                                         const uint8_t* __restrict__ arena,
-                                                        double* __restrict__ partials, int csplit) {
+                                                        double* __restrict__ partials, int csplit,
+                                                        int nsmall) {
     constexpr int TS = kMxTile;
     constexpr int grp = map_group(0, sizeof(ST) == 2, SP::kParts == 3);
-    __shared__ MxLds<SP::kParts> L;
+    __shared__ union {
+        MxLds<SP::kParts> mx;
+        SmallLds small;
+    } lds;
+    if ((int)blockIdx.x < nsmall) {
+        map_small_tile<ST>(lds.small, pairs, order_seg, order_start, hdr, arena, partials, blockIdx.x);
+        return;
+    }
+    MxLds<SP::kParts>& L = lds.mx;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, j = lane & 15;
     if (tid == 0) {
@@ -638,7 +651,7 @@ __global__ __launch_bounds__(256, SP::kParts == 2 ? 4 : 2) void map_mx_kernel(co
     // with xcd_block, so that the workgroups of one XCD hold one contiguous
     // range of tiles. A smaller, persistent grid takes its work items from the
     // per-XCD dynamic queue.
-    const int nwg = gridDim.x;
+    const int nwg = gridDim.x - nsmall;
     const int ntl = t_end - t_begin;
     const int nwork = ntl * csplit;
     const bool persistent = nwg < nwork;
@@ -646,7 +659,7 @@ __global__ __launch_bounds__(256, SP::kParts == 2 ? 4 : 2) void map_mx_kernel(co
     __shared__ int s_tile;
     // (with more workgroups than work items, item floor(v n / nwg) of virtual
     // workgroup v, so that every XCD still gets work)
-    const int vb = xcd_block(blockIdx.x, nwg);
+    const int vb = xcd_block(blockIdx.x - nsmall, nwg);
     int next = (int)(((int64_t)vb * nwork) / nwg);
     const int w_hi = (int)(((int64_t)(vb + 1) * nwork) / nwg);
     for (;;) {
@@ -711,7 +724,32 @@ __global__ __launch_bounds__(256, SP::kParts == 2 ? 4 : 2) void map_mx_kernel(co
     }
 }
 
-hipError_t launch_map_mx(bool half, bool exact, int grid, const PairDev* pairs, const int32_t* order_seg,
+// The FP64 tiles by themselves, for grids of a fixed size (capture, persistent).
+template <typename ST>
+__global__ __launch_bounds__(256) void map_small_kernel(const PairDev* __restrict__ pairs,
+                                                        const int32_t* __restrict__ order_seg,
+                                                        const int32_t* __restrict__ order_start,
+                                                        const BatchHdr* __restrict__ hdr,
+                                                        const uint8_t* __restrict__ arena,
+                                                        double* __restrict__ partials) {
+    __shared__ SmallLds L;
+    const int n = 3 * hdr->tiles[map_group(1, sizeof(ST) == 2)];
+    for (int item = blockIdx.x; item < n; item += gridDim.x) {
+        map_small_tile<ST>(L, pairs, order_seg, order_start, hdr, arena, partials, item);
+        __syncthreads();
+    }
+}
+
+hipError_t launch_map_small(bool half, int grid, const PairDev* pairs, const int32_t* order_seg,
+                            const int32_t* order_start, const BatchHdr* hdr, const void* arena, double* partials,
+                            hipStream_t st) {
+    const uint8_t* a = reinterpret_cast<const uint8_t*>(arena);
+    if (half) map_small_kernel<__half><<<grid, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials);
+    else map_small_kernel<float><<<grid, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials);
+    return hipGetLastError();
+}
+
+hipError_t launch_map_mx(bool half, bool exact, int grid, int nsmall, const PairDev* pairs, const int32_t* order_seg,
                          const int32_t* order_start, const BatchHdr* hdr, const void* arena, double* partials,
                          int csplit, hipStream_t st) {
     if (csplit != 1 && csplit != 3) return hipErrorInvalidValue;
@@ -719,11 +757,11 @@ hipError_t launch_map_mx(bool half, bool exact, int grid, const PairDev* pairs, 
     // float RGB input may hold any value: the exact split; every other format
     // gives bounded XYB values: the scaled fp16 split
     if (exact) {
-        if (half) map_mx_kernel<__half, SplitBf16x3><<<grid, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit);
-        else map_mx_kernel<float, SplitBf16x3><<<grid, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit);
+        if (half) map_mx_kernel<__half, SplitBf16x3><<<grid + nsmall, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit, nsmall);
+        else map_mx_kernel<float, SplitBf16x3><<<grid + nsmall, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit, nsmall);
     } else {
-        if (half) map_mx_kernel<__half, SplitF16x2><<<grid, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit);
-        else map_mx_kernel<float, SplitF16x2><<<grid, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit);
+        if (half) map_mx_kernel<__half, SplitF16x2><<<grid + nsmall, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit, nsmall);
+        else map_mx_kernel<float, SplitF16x2><<<grid + nsmall, 256, 0, st>>>(pairs, order_seg, order_start, hdr, a, partials, csplit, nsmall);
     }
     return hipGetLastError();
 }

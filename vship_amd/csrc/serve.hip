@@ -73,7 +73,7 @@ public:
                        : default_map_th(cfg_.max_width, cfg_.max_height);
         // the budget covers the arenas of both in-flight steps
         o.arena_bytes = (int64_t)(cfg_.memory_budget / 2);
-        o.max_map_tiles = (int64_t)cfg_.max_pairs_per_step * map_tiles(cfg_.max_width, cfg_.max_height, 32);
+        o.max_map_tiles = (int64_t)cfg_.max_pairs_per_step * max_map_tiles(cfg_.max_width, cfg_.max_height);
         o.persistent_grid = cfg_.persistent_grid;
         o.use_graph = cfg_.use_graph != 0;
         step_budget_ = o.arena_bytes;

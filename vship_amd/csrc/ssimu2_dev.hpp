@@ -97,7 +97,8 @@ struct BatchHdr {
     // Map segments (one per pair and scale) fall in two classes: class 0
     // accumulates the moment blur in FP32, class 1 (segments of fewer than
     // kSmallSegment pixels, where FP32 rounding noise would not average out)
-    // in FP64 with tiles of kSmallTH rows. Each class splits by plane storage
+    // in FP64 with tiles of kSmallTH rows (beside the matrix-core kernel, tiles
+    // of kSmallTile x kSmallTile). Each class splits by plane storage
     // into group 2*class (FP32 planes) and 2*class+1 (FP16 planes). On the
     // matrix cores, class-0 segments of pairs with float RGB input go to
     // groups 4 (FP32 planes) and 5 (FP16 planes) instead: they take the exact
@@ -127,8 +128,19 @@ constexpr int kSmallTH = 48;
 constexpr int kMapMfma = 1;
 constexpr int kMxTile = 64;
 constexpr int kMxTileH = 128;
-__host__ __device__ constexpr int map_tile_w(int th) { return th == kMapMfma ? kMxTile : kMapTW; }
-__host__ __device__ constexpr int map_tile_h(int th) { return th == kMapMfma ? kMxTileH : th; }
+// Tile height value of the FP64 class beside the matrix-core kernel: tiles of
+// kSmallTile x kSmallTile. A segment of fewer than kSmallSegmentMx pixels has
+// at most 256 of them (one pixel wide), and a pair's segments, each of half the
+// one before, at most kSmallTilesMax.
+constexpr int kMapSmall = 2;
+constexpr int kSmallTile = 16;
+constexpr int kSmallTilesMax = 512;
+__host__ __device__ constexpr int map_tile_w(int th) {
+    return th == kMapMfma ? kMxTile : th == kMapSmall ? kSmallTile : kMapTW;
+}
+__host__ __device__ constexpr int map_tile_h(int th) {
+    return th == kMapMfma ? kMxTileH : th == kMapSmall ? kSmallTile : th;
+}
 
 // The 17-tap Gaussian (sigma 1.5, radius 8) of src/ssimu2/gaussianblur.hpp:7-18
 // and src/util/preprocessor.hpp:89-92, normalised to sum 1 and rounded to

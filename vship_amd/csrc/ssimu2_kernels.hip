@@ -778,59 +778,84 @@ __constant__ double kWeights[108] = {
     0.0, 0.0, 0.0, 0.0005130064588990679, 0.0, 0.00010854057858411537,
 };
 
-__device__ double ssimu2_score_from_features(const double* f) {
-    double s = 0.0;
-    for (int i = 0; i < 108; i++) s = fma(kWeights[i], f[i], s);
+__device__ double ssimu2_score(double s) {
     s *= 0.9562382616834844;
     s = (6.248496625763138e-5 * s * s) * s + 2.326765642916932 * s - 0.020884521182843837 * s * s;
     return s > 0.0 ? 100.0 - 10.0 * pow(s, 0.6276336467831387) : 100.0;
 }
 
-__global__ __launch_bounds__(256) void finalize_kernel(const PairDev* __restrict__ pairs,
-                                                       const int32_t* __restrict__ seg_start,
-                                                       const int32_t* __restrict__ seg_count,
-                                                       const BatchHdr* __restrict__ hdr,
-                                                       const double* __restrict__ partials,
-                                                       double* __restrict__ scores, double* __restrict__ features) {
-    __shared__ double part[14][kFeat];
+// A workgroup per pair. Latency is all its time, so nothing waits in turn: the
+// six segments' partials are loaded together (group g of kFinGroups sums tiles
+// g, g + kFinGroups, ... of each segment, in order), eight lanes add the
+// groups' sums of a feature, and one wave the weighted features. With a thread
+// per group and feature of one segment after the other, and one thread for
+// the weights, it took 13.1 us for a 1920 x 1080 pair (9.5 for a 256 x 256 one); now 6.5 (4.8).
+constexpr int kFinGroups = 56, kFinThreads = 1024;
+static_assert(kFinGroups * kFeat <= kFinThreads && kFinGroups % 8 == 0 && 8 * kScales * kFeat <= kFinThreads,
+              "threads of the finalize kernel");
+
+__global__ __launch_bounds__(kFinThreads) void finalize_kernel(const PairDev* __restrict__ pairs,
+                                                               const int32_t* __restrict__ seg_start,
+                                                               const int32_t* __restrict__ seg_count,
+                                                               const BatchHdr* __restrict__ hdr,
+                                                               const double* __restrict__ partials,
+                                                               double* __restrict__ scores,
+                                                               double* __restrict__ features) {
+    __shared__ double part[kScales][kFinGroups][kFeat];
     __shared__ double feat[108];
     const int tid = threadIdx.x;
     const int npairs = hdr->npairs;
     for (int p = blockIdx.x; p < npairs; p += gridDim.x) {
         const PairDev& P = pairs[p];
-        for (int s = 0; s < kScales; s++) {
-            const int t0 = seg_start[p * kScales + s], t1 = t0 + seg_count[p * kScales + s];
-            if (tid < 14 * kFeat) {
-                const int k = tid % kFeat, g = tid / kFeat;
-                // tiles t0 + g, t0 + g + 14, ... summed in that order; the
-                // loads go eight at a time, so that one wait covers eight
-                // tiles instead of one
-                const int n = t0 + g < t1 ? (t1 - t0 - g + 13) / 14 : 0;
-                const double* src = partials + (int64_t)(t0 + g) * kFeat + k;
-                double a = 0.0;
-                for (int i = 0; i < n; i += 8) {
+        if (tid < kFinGroups * kFeat) {
+            const int k = tid % kFeat, g = tid / kFeat;
+            double a[kScales];
+            int n[kScales];
+            const double* src[kScales];
+#pragma unroll
+            for (int s = 0; s < kScales; s++) {
+                const int count = seg_count[p * kScales + s] - g;
+                n[s] = count > 0 ? (count + kFinGroups - 1) / kFinGroups : 0;
+                src[s] = partials + (int64_t)(seg_start[p * kScales + s] + g) * kFeat + k;
+                a[s] = n[s] > 0 ? src[s][0] : 0.0;
+            }
+            // the rest of the larger segments, eight loads at a time
+#pragma unroll
+            for (int s = 0; s < kScales; s++) {
+                for (int i = 1; i < n[s]; i += 8) {
                     double v[8];
 #pragma unroll
-                    for (int u = 0; u < 8; u++) v[u] = i + u < n ? src[(int64_t)(i + u) * 14 * kFeat] : 0.0;
+                    for (int u = 0; u < 8; u++) v[u] = i + u < n[s] ? src[s][(int64_t)(i + u) * kFinGroups * kFeat] : 0.0;
 #pragma unroll
                     for (int u = 0; u < 8; u++)
-                        if (i + u < n) a += v[u];
+                        if (i + u < n[s]) a[s] += v[u];
                 }
-                part[g][k] = a;
+                part[s][g][k] = a[s];
             }
-            __syncthreads();
-            if (tid < kFeat) {
-                double a = 0.0;
-                for (int g = 0; g < 14; g++) a += part[g][tid];
-                const double n = (double)P.sw[s] * (double)P.sh[s];
-                const int c = tid / 6, mnorm = tid % 6, m = mnorm >> 1, nrm = mnorm & 1;
-                const double mean = a / n;
+        }
+        __syncthreads();
+        if (tid < 8 * kScales * kFeat) {
+            const int f = tid >> 3, s = f / kFeat, k = f % kFeat;
+            double a = 0.0;
+#pragma unroll
+            for (int g = 0; g < kFinGroups / 8; g++) a += part[s][8 * g + (tid & 7)][k];
+#pragma unroll
+            for (int off = 1; off < 8; off <<= 1) a += __shfl_xor(a, off, 64);
+            if ((tid & 7) == 0) {
+                const double mean = a / ((double)P.sw[s] * (double)P.sh[s]);
+                const int c = k / 6, m = (k % 6) >> 1, nrm = k & 1;
                 feat[c * 36 + s * 6 + nrm * 3 + m] = nrm ? sqrt(sqrt(mean)) : mean;
             }
-            __syncthreads();
         }
-        if (tid == 0) scores[p] = ssimu2_score_from_features(feat);
+        __syncthreads();
         if (features && tid < 108) features[(int64_t)p * 108 + tid] = feat[tid];
+        if (tid < 64) {
+            double s = kWeights[tid] * feat[tid];
+            if (tid < 44) s = fma(kWeights[64 + tid], feat[64 + tid], s);
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+            if (tid == 0) scores[p] = ssimu2_score(s);
+        }
         __syncthreads();
     }
 }
@@ -882,7 +907,7 @@ hipError_t launch_map(bool half, int cls, int th, int grid, const PairDev* pairs
 hipError_t launch_finalize(int grid, const PairDev* pairs, const int32_t* seg_start, const int32_t* seg_count,
                            const BatchHdr* hdr, const double* partials, double* scores, double* features,
                            hipStream_t st) {
-    finalize_kernel<<<grid, 256, 0, st>>>(pairs, seg_start, seg_count, hdr, partials, scores, features);
+    finalize_kernel<<<grid, kFinThreads, 0, st>>>(pairs, seg_start, seg_count, hdr, partials, scores, features);
     return hipGetLastError();
 }
 

@@ -118,7 +118,7 @@ Vship_Exception Vship_SSIMU2BatchTune(const Vship_SSIMU2Pair* pairs, int npairs,
                     o.fp16 = fp16_planes != 0;
                     o.map_th = th;
                     o.arena_bytes = arena;
-                    o.max_map_tiles = (int64_t)npairs * map_tiles(mw, mh, 32);  // bound for every shape
+                    o.max_map_tiles = (int64_t)npairs * max_map_tiles(mw, mh);  // bound for every shape
                     o.persistent_grid = grids[gi];
                     o.use_graph = graph != 0;
                     Engine e(o);

@@ -97,7 +97,7 @@ FrameHandle::FrameHandle(int w, int h, int device) : width(w), height(h), device
     o.max_pairs = 1;
     o.map_th = default_map_th(w, h);
     o.arena_bytes = pair_bytes(w, h, false);
-    o.max_map_tiles = map_tiles(w, h, 32);
+    o.max_map_tiles = max_map_tiles(w, h);
     // one 1080p float plane is 8.3 MB: 4 MiB chunks keep two of them in
     // flight per plane while the next one is copied in
     o.host_chunk_bytes = 4ll << 20;
@@ -608,7 +608,7 @@ Vship_Exception Vship_SSIMU2BatchInit(Vship_SSIMU2BatchHandler* handler, const V
                                          : (int64_t)cfg->max_pairs *
                                                (int64_t)Vship_SSIMU2PairFootprint(cfg->max_width, cfg->max_height,
                                                                                   cfg->fp16_planes);
-        o.max_map_tiles = (int64_t)cfg->max_pairs * map_tiles(cfg->max_width, cfg->max_height, 32);
+        o.max_map_tiles = (int64_t)cfg->max_pairs * max_map_tiles(cfg->max_width, cfg->max_height);
         o.use_graph = cfg->use_graph != 0;  // a captured graph runs a fixed grid (4 x CUs when 0)
         o.profile = cfg->profile != 0;
         o.host_copy_threads = 4;
