@@ -514,17 +514,23 @@ void Engine::submit_host(const PairInput* pairs, int n) {
         HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&in_d_[k]), U.total), E_OutOfVRAM);
         in_cap_[k] = U.total;
     }
-    // the upload into buffer k starts after the kernels that read it last
-    HIP_OR_THROW(hipStreamWaitEvent(copy_, in_free_[k], 0), E_BadDeviceCode);
-    stager_->upload(in_d_[k], U, copy_);
+    // Without threads of its own (a per-frame handle, whose caller waits for
+    // each pair) the stager works in the kernels' stream; else the upload runs
+    // beside the previous batch's kernels, into buffer k after those that read
+    // it last.
+    const bool same = opt_.host_copy_threads == 0;
+    if (!same) HIP_OR_THROW(hipStreamWaitEvent(copy_, in_free_[k], 0), E_BadDeviceCode);
+    stager_->upload(in_d_[k], U, same ? stream_ : copy_);
     std::vector<PairInput> dev(pairs, pairs + n);
     for (int i = 0; i < n; i++)
         for (int im = 0; im < 2; im++)
             for (int pl = 0; pl < 3; pl++) dev[i].src[im][pl] = in_d_[k] + U.off[(size_t)i * 6 + im * 3 + pl];
-    HIP_OR_THROW(hipEventRecord(in_ready_[k], copy_), E_BadDeviceCode);
-    HIP_OR_THROW(hipStreamWaitEvent(stream_, in_ready_[k], 0), E_BadDeviceCode);
+    if (!same) {
+        HIP_OR_THROW(hipEventRecord(in_ready_[k], copy_), E_BadDeviceCode);
+        HIP_OR_THROW(hipStreamWaitEvent(stream_, in_ready_[k], 0), E_BadDeviceCode);
+    }
     submit(dev.data(), n);
-    HIP_OR_THROW(hipEventRecord(in_free_[k], stream_), E_BadDeviceCode);
+    if (!same) HIP_OR_THROW(hipEventRecord(in_free_[k], stream_), E_BadDeviceCode);
 }
 
 void Engine::set_host_staging(int64_t chunk_bytes, int slots, int copy_threads) {

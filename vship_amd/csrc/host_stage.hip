@@ -3,6 +3,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
+#include <thread>
 
 #include "engine.hpp"
 
@@ -65,7 +67,52 @@ UploadPlan plan_upload(const uint8_t* const* src, const size_t* bytes, int n) {
     return P;
 }
 
-HostStager::HostStager(int device, size_t chunk_bytes, int slots, int threads) {
+namespace {
+
+// The helpers of the stagers without threads of their own. Three beside the
+// caller saturate PCIe from pageable memory (a CPU thread copies about 25 GB/s of its
+// 57), and as there is one team, many handles on many threads still make only
+// three extra threads: one upload has them, the others copy alone.
+std::shared_ptr<CopyTeam> shared_team() {
+    static std::mutex mu;
+    static std::weak_ptr<CopyTeam> team;
+    std::lock_guard<std::mutex> lk(mu);
+    std::shared_ptr<CopyTeam> t = team.lock();
+    if (!t) {
+        const int cpus = (int)std::thread::hardware_concurrency();
+        t = std::make_shared<CopyTeam>(std::min(3, std::max(0, cpus - 1)));
+        team = t;
+    }
+    return t;
+}
+
+// Bytes between a chunk of the ring and device memory, by a kernel in the
+// stream itself: a DMA and its hand-over to the kernels behind it cost about
+// 20 us each besides the bytes (measured at 1, 2 and 4 MiB), more than a small
+// picture's whole upload. Bound by PCIe; 64 workgroups keep 256 KiB of 16-byte
+// accesses in flight, several times what the link's latency needs.
+constexpr int kMoveGroups = 64;
+__global__ __launch_bounds__(256) void move_kernel(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src,
+                                                   size_t bytes) {
+    const size_t n16 = bytes / 16, step = (size_t)gridDim.x * 256, t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = t; i < n16; i += step)
+        reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    for (size_t i = 16 * n16 + t; i < bytes; i += step) dst[i] = src[i];
+}
+
+// dst and src 16-byte aligned, one of them in page-locked memory
+void move_chunk(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    const int groups = (int)std::min<size_t>(kMoveGroups, (bytes / 16 + 255) / 256 + 1);
+    move_kernel<<<groups, 256, 0, st>>>(static_cast<uint8_t*>(dst), static_cast<const uint8_t*>(src), bytes);
+    HIP_OR_THROW(hipGetLastError(), E_BadDeviceCode);
+}
+
+constexpr size_t kPiece = 256 << 10;     // bytes a thread copies at a time
+constexpr size_t kSharedMin = 1 << 20;   // below it, waking the helpers costs more than it saves
+
+}  // namespace
+
+HostStager::HostStager(int device, size_t chunk_bytes, int slots, int threads) : shared_(threads == 0) {
     HIP_OR_THROW(hipSetDevice(device), E_BadDeviceArgument);
     chunk_ = std::max<size_t>(chunk_bytes / 4096 * 4096, 4096);
     slots = std::max(slots, 2);
@@ -109,6 +156,7 @@ void HostStager::upload(void* dst, const void* src, size_t bytes, hipStream_t st
 
 void HostStager::upload(uint8_t* dst_base, const UploadPlan& plan, hipStream_t st) {
     if (!dst_base) VSHIP_THROW(E_BadPointer);
+    if (shared_) return upload_shared(dst_base, plan, st);
     // the open chunk: slot k holds device bytes [c0, c0 + fill)
     int k = -1;
     size_t c0 = 0, fill = 0;
@@ -153,6 +201,60 @@ void HostStager::upload(uint8_t* dst_base, const UploadPlan& plan, hipStream_t s
     flush();
 }
 
+CopyTeam& HostStager::team_for(size_t bytes) {
+    static CopyTeam nobody(0);
+    if (!shared_ || bytes < kSharedMin) return nobody;
+    if (!team_) team_ = shared_team();
+    return *team_;
+}
+
+void HostStager::upload_shared(uint8_t* dst_base, const UploadPlan& plan, hipStream_t st) {
+    // chunks of the ring, each a device range of whole or partial runs
+    struct Chunk {
+        size_t off, bytes;
+    };
+    std::vector<Chunk> chunks;
+    std::vector<CopyTeam::Piece> pieces;
+    bool open = false;  // the last chunk may take the next run (no page-locked run lies between)
+    for (const UploadPlan::Run& r : plan.runs) {
+        if (r.locked) {
+            HIP_OR_THROW(hipMemcpyAsync(dst_base + r.off, r.src, r.bytes, hipMemcpyHostToDevice, st), E_BadPointer);
+            direct_bytes_ += r.bytes;
+            open = false;
+            continue;
+        }
+        for (size_t done = 0; done < r.bytes;) {
+            const size_t dpos = r.off + done;
+            if (!open || dpos >= chunks.back().off + chunk_) chunks.push_back({dpos, 0});
+            open = true;
+            Chunk& c = chunks.back();
+            const size_t n = std::min({r.bytes - done, c.off + chunk_ - dpos, kPiece});
+            const int slot = (next_ + (int)chunks.size() - 1) % (int)ring_.size();
+            pieces.push_back({ring_[slot] + (dpos - c.off), r.src + done, n, (int)chunks.size() - 1});
+            c.bytes = dpos - c.off + n;
+            done += n;
+        }
+        pageable_bytes_ += r.bytes;
+    }
+    if (chunks.empty()) return;
+    const int nslots = (int)ring_.size(), n = (int)chunks.size(), first = next_;
+    next_ = (first + n) % nslots;
+    team_for(plan.total).run(
+        pieces, n, nslots,
+        [&](int c, bool wait) {
+            // the slot's previous DMA has to have read it before it is refilled
+            hipEvent_t e = ev_[(first + c) % nslots];
+            if (!wait) return hipEventQuery(e) == hipSuccess;
+            HIP_OR_THROW(hipEventSynchronize(e), E_BadDeviceCode);
+            return true;
+        },
+        [&](int c) {
+            const int k = (first + c) % nslots;
+            move_chunk(dst_base + chunks[c].off, ring_[k], chunks[c].bytes, st);
+            HIP_OR_THROW(hipEventRecord(ev_[k], st), E_BadDeviceCode);
+        });
+}
+
 void HostStager::download_rows(void* dst, int64_t dst_stride, const void* src, int64_t src_stride,
                                size_t row_bytes, int rows, hipStream_t st) {
     if (rows < 1 || row_bytes == 0) return;
@@ -169,7 +271,12 @@ void HostStager::download_rows(void* dst, int64_t dst_stride, const void* src, i
         direct_bytes_ += row_bytes * rows;
         return;
     }
-    if (row_bytes > chunk_) VSHIP_THROW(E_BadPointer);
+    if (row_bytes > chunk_) {  // a row of over half a million samples
+        HIP_OR_THROW(hipStreamSynchronize(st), E_BadPointer);
+        HIP_OR_THROW(hipMemcpy2D(d, dst_stride, s, src_stride, row_bytes, rows, hipMemcpyDeviceToHost), E_BadPointer);
+        pageable_bytes_ += row_bytes * rows;
+        return;
+    }
     const int per = (int)std::min<size_t>(chunk_ / row_bytes, (size_t)rows);
     const int nchunks = (rows + per - 1) / per;
     const int nslots = (int)ring_.size();
@@ -178,22 +285,42 @@ void HostStager::download_rows(void* dst, int64_t dst_stride, const void* src, i
         const int k = (next_ + c) % nslots;
         const int r0 = c * per, n = std::min(per, rows - r0);
         HIP_OR_THROW(hipEventSynchronize(ev_[k]), E_BadDeviceCode);
-        HIP_OR_THROW(hipMemcpy2DAsync(ring_[k], row_bytes, s + (int64_t)r0 * src_stride, src_stride, row_bytes, n,
-                                      hipMemcpyDeviceToHost, st),
-                     E_BadPointer);
+        const uint8_t* from = s + (int64_t)r0 * src_stride;
+        if (shared_ && src_stride == (int64_t)row_bytes && reinterpret_cast<uintptr_t>(from) % 16 == 0)
+            move_chunk(ring_[k], from, row_bytes * n, st);
+        else
+            HIP_OR_THROW(hipMemcpy2DAsync(ring_[k], row_bytes, from, src_stride, row_bytes, n, hipMemcpyDeviceToHost, st),
+                         E_BadPointer);
         HIP_OR_THROW(hipEventRecord(ev_[k], st), E_BadDeviceCode);
     };
     for (int c = 0; c < std::min(nchunks, nslots); c++) enqueue(c);
-    for (int c = 0; c < nchunks; c++) {
-        const int k = (next_ + c) % nslots;
-        const int r0 = c * per, n = std::min(per, rows - r0);
-        HIP_OR_THROW(hipEventSynchronize(ev_[k]), E_BadDeviceCode);
-        if (dst_stride == (int64_t)row_bytes)
-            std::memcpy(d + (int64_t)r0 * dst_stride, ring_[k], row_bytes * n);
-        else
-            for (int r = 0; r < n; r++) std::memcpy(d + (int64_t)(r0 + r) * dst_stride, ring_[k] + row_bytes * r, row_bytes);
+    // pieces of whole rows, copied out of a chunk once its DMA has arrived
+    std::vector<CopyTeam::Piece> pieces;
+    const int piece_rows = std::max(1, (int)(kPiece / row_bytes));
+    for (int c = 0; c < nchunks; c++)
+        for (int r = c * per; r < std::min(rows, (c + 1) * per); r += piece_rows) {
+            const int n = std::min(piece_rows, std::min(rows, (c + 1) * per) - r);
+            CopyTeam::Piece p{d + (int64_t)r * dst_stride, ring_[(next_ + c) % nslots] + row_bytes * (r - c * per),
+                              row_bytes, c};
+            if (dst_stride == (int64_t)row_bytes) {
+                p.bytes = row_bytes * n;
+            } else {
+                p.rows = n;
+                p.dst_stride = dst_stride;
+                p.src_stride = (int64_t)row_bytes;
+            }
+            pieces.push_back(p);
+        }
+    auto arrived = [&](int c, bool wait) {
+        hipEvent_t e = ev_[(next_ + c) % nslots];
+        if (!wait) return hipEventQuery(e) == hipSuccess;
+        HIP_OR_THROW(hipEventSynchronize(e), E_BadDeviceCode);
+        return true;
+    };
+    auto copied = [&](int c) {
         if (c + nslots < nchunks) enqueue(c + nslots);
-    }
+    };
+    team_for(row_bytes * rows).run(pieces, nchunks, nslots, arrived, copied);
     next_ = (next_ + nchunks) % nslots;
     pageable_bytes_ += row_bytes * rows;
 }

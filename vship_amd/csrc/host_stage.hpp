@@ -16,6 +16,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "parallel_copy.hpp"
@@ -53,6 +54,9 @@ UploadPlan plan_upload(const uint8_t* const* src, const size_t* bytes, int n);
 
 class HostStager {
 public:
+    // threads: the CPU threads that copy pageable memory, the caller among them;
+    // 0: the caller and, where they are free, the helpers that all such stagers
+    // of the process share (kept while one of them exists)
     HostStager(int device, size_t chunk_bytes, int slots, int threads);
     ~HostStager();
     HostStager(const HostStager&) = delete;
@@ -84,12 +88,16 @@ public:
 
 private:
     void release();
+    void upload_shared(uint8_t* dst_base, const UploadPlan& plan, hipStream_t st);
+    CopyTeam& team_for(size_t bytes);  // who copies that many pageable bytes
 
     size_t chunk_ = 0;
     std::vector<uint8_t*> ring_;  // page-locked chunks
     std::vector<hipEvent_t> ev_;  // slot i's last DMA
     int next_ = 0;
     ParallelCopy* pool_ = nullptr;
+    bool shared_ = false;
+    std::shared_ptr<CopyTeam> team_;
     uint64_t pageable_bytes_ = 0, direct_bytes_ = 0;
 };
 

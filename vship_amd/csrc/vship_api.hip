@@ -91,6 +91,10 @@ void gpu_full_check(int gpu_id) {
 // ---------------------------------------------------------------------------
 // per-frame handles (Vship_SSIMU2Handler)
 // ---------------------------------------------------------------------------
+// staging ring of a per-frame handle (both metrics)
+constexpr int64_t kFrameChunk = 2ll << 20;
+constexpr int kFrameSlots = 8;
+
 FrameHandle::FrameHandle(int w, int h, int device) : width(w), height(h), device(device) {
     EngineOptions o;
     o.device = device;
@@ -98,11 +102,11 @@ FrameHandle::FrameHandle(int w, int h, int device) : width(w), height(h), device
     o.map_th = default_map_th(w, h);
     o.arena_bytes = pair_bytes(w, h, false);
     o.max_map_tiles = max_map_tiles(w, h);
-    // one 1080p float plane is 8.3 MB: 4 MiB chunks keep two of them in
-    // flight per plane while the next one is copied in
-    o.host_chunk_bytes = 4ll << 20;
-    o.host_slots = 4;
-    o.host_copy_threads = 1;  // frame-level parallelism comes from the callers' threads
+    // a frame's planes go in several chunks, so that the first cross PCIe while
+    // the last are copied in
+    o.host_chunk_bytes = kFrameChunk;
+    o.host_slots = kFrameSlots;
+    o.host_copy_threads = 0;  // the helpers that all per-frame handles share, where they are free
     engine = std::make_unique<Engine>(o);
 }
 
@@ -141,7 +145,7 @@ double FrameHandle::compute(int fmt, const uint8_t* const p1[3], const uint8_t* 
 // ---------------------------------------------------------------------------
 ButterHandle::ButterHandle(int w, int h, int qnorm, float intensity, int dev) : width(w), height(h), device(dev) {
     engine = std::make_unique<bt::Engine>(w, h, 1, qnorm, intensity, dev);
-    stager = std::make_unique<HostStager>(dev, (size_t)4 << 20, 4, 1);
+    stager = std::make_unique<HostStager>(dev, (size_t)kFrameChunk, kFrameSlots, 0);
     HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&map), sizeof(float) * (size_t)w * h), E_OutOfVRAM);
 }
 
@@ -160,29 +164,31 @@ void ButterHandle::compute(int fmt, const uint8_t* const p1[3], const uint8_t* c
     if (dst && dst_stride < (int64_t)width * 4) VSHIP_THROW(E_BadPointer);
     // each plane is one contiguous block of (height - 1) strides plus a row
     const size_t blk1 = (size_t)s1 * (height - 1) + row, blk2 = (size_t)s2 * (height - 1) + row;
-    const size_t a1 = (blk1 + 255) / 256 * 256, a2 = (blk2 + 255) / 256 * 256;
-    const size_t need = 3 * (a1 + a2);
+    const uint8_t* src[6];
+    size_t blk[6];
+    for (int pl = 0; pl < 3; pl++) {
+        src[pl] = p1[pl];
+        src[3 + pl] = p2[pl];
+        blk[pl] = blk1;
+        blk[3 + pl] = blk2;
+    }
     HIP_OR_THROW(hipSetDevice(device), E_BadDeviceArgument);
-    if (need > staging_bytes) {
+    const UploadPlan U = plan_upload(src, blk, 6);
+    if (U.total > staging_bytes) {
         if (staging) (void)hipFree(staging);
         staging = nullptr;
         staging_bytes = 0;
-        HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&staging), need), E_OutOfVRAM);
-        staging_bytes = need;
+        HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&staging), U.total), E_OutOfVRAM);
+        staging_bytes = U.total;
     }
     hipStream_t st = engine->stream();
+    stager->upload(staging, U, st);
     bt::PairDesc d{};
-    for (int im = 0; im < 2; im++) {
-        const uint8_t* const* src = im == 0 ? p1 : p2;
-        const int64_t sp = im == 0 ? s1 : s2;
-        const size_t blk = im == 0 ? blk1 : blk2;
+    for (int im = 0; im < 2; im++)
         for (int pl = 0; pl < 3; pl++) {
-            uint8_t* dstp = staging + (im == 0 ? pl * a1 : 3 * a1 + pl * a2);
-            stager->upload(dstp, src[pl], blk, st);
-            d.src[im][pl] = dstp;
-            d.stride[im][pl] = sp;
+            d.src[im][pl] = staging + U.off[3 * im + pl];
+            d.stride[im][pl] = im == 0 ? s1 : s2;
         }
-    }
     d.map = dst ? map : nullptr;
     d.map_stride = (int64_t)width * 4;
     engine->run(fmt, &d, 1, norms);
