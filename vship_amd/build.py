@@ -30,12 +30,11 @@ HIPFLAGS = [
     "-I", os.path.join(ROOT, "include"),
 ]
 # Per-source options. The matrix-core map kernel is scheduled by LLVM's
-# memory-clause strategy: measured at 1920x1080, 240 pairs, 7.59-7.61 ms
-# against 7.67-7.72 ms with the default (occupancy) strategy on one box, the
-# same scores; the ILP strategy gave 7.53-7.64 ms and the iterative
-# register-minimising one 9.26 ms.
+# iterative ILP strategy: 240 pairs of 1920x1080 in 11.09 ms, against 11.12 with
+# the memory-clause strategy, 11.15 with the default and 11.20 with the plain
+# ILP one, the same scores; 24 4K pairs 3.60, 3.64, 3.66 and 3.63.
 SOURCE_FLAGS = {
-    "map_mfma.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],
+    "map_mfma.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
 }
 LIB = os.path.join(HERE, "libvship.so")
 SYNTH_SRC = os.path.join(HERE, "synth", "synth.c")

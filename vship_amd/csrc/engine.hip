@@ -347,17 +347,31 @@ PlanInfo plan_batch(const PairInput* in, int n, int max_pairs, bool fp16, int ma
     return P;
 }
 
+// How a launch of the matrix-core map kernel shares its tiles out (launch_map_mx):
+// the fewer, the finer. Fewer than four tiles per CU: a workgroup per channel, a
+// wave per half of a tile's rows (one 1080p pair, 379 tiles, 88 us; a wave for
+// all rows 95; three pairs 189 either way, four 238 and 229). Fewer than 128 per
+// CU: a workgroup per channel (eight pairs 488 us, a workgroup per tile 494; 48
+// pairs, 18,192 tiles, 2,165 and 2,198; but 240 pairs 11,137 and 11,039).
+struct MapSplit {
+    int rows, csplit;
+};
+static MapSplit map_split(int tiles, bool eager, int num_cus) {
+    if (!eager || tiles >= 128 * num_cus) return {1, 1};
+    return {tiles < 4 * num_cus ? 2 : 1, 3};
+}
+
 void launch_batch(const DescView& d, const PlanInfo& P, const LaunchShape& S, void* arena, double* partials,
                   double* scores, double* features, const Taps& taps, hipStream_t st, hipEvent_t* ev) {
     const bool graph = S.graph;
     const int fixed = S.persistent_grid > 0 ? S.persistent_grid : 4 * S.num_cus;
-    auto grid_for = [&](int work, int cap_in_graph) {
+    auto grid_for = [&](int work, int persistent, int cap_in_graph) {
         if (graph) return cap_in_graph;
-        if (S.persistent_grid > 0) return std::max(1, std::min(work, fixed));
+        if (S.persistent_grid > 0) return std::max(1, std::min(work, persistent));
         return std::max(1, work);
     };
-    const int g_prep = grid_for(P.ntiles_prep, fixed);
-    const int g_fin = grid_for(P.npairs, std::min(S.max_pairs, fixed));
+    const int g_prep = grid_for(P.ntiles_prep, fixed, fixed);
+    const int g_fin = grid_for(P.npairs, fixed, std::min(S.max_pairs, fixed));
     // pairs on the generic chroma path have their own prep kernel, and a batch
     // of only such pairs no other; a captured graph always holds both (each
     // returns at once when the batch has none of its pairs)
@@ -369,45 +383,42 @@ void launch_batch(const DescView& d, const PlanInfo& P, const LaunchShape& S, vo
     // one launch per map group; FP16-plane groups exist only with FP16 storage,
     // and an eager launch is skipped when its group is empty
     const bool mfma = S.map_th == kMapMfma;
-    // An eager launch of the matrix-core kernel brings the FP64 tiles of its
-    // plane storage along, a workgroup per tile and channel ahead of its own:
-    // by themselves these few workgroups, whose time is latency, held the GPU
-    // for 14 us of a 1920 x 1080 pair's 116.
-    const bool merged = mfma && !graph && S.persistent_grid == 0;
-    int small[2] = {};  // FP64 workgroups still to be launched, by plane storage
-    if (merged)
-        for (int half = 0; half < 2; half++) small[half] = 3 * P.ntiles_grp[map_group(1, half)];
+    // An eager launch of few tiles splits them: on the matrix-core kernel by
+    // map_split, and for the vector kernels (as few as 1 workgroup per CU in the
+    // FP64 class) a workgroup per channel when these fit in two rounds, as for
+    // one pair per call. The partials are the same.
+    // The matrix-core kernel's launch of the fewest tiles also brings the FP64
+    // tiles of its plane storage along, a workgroup per tile and channel ahead of
+    // its own: by themselves these few workgroups, whose time is latency, held
+    // the GPU for 14 us of a 1920 x 1080 pair's 116.
+    const bool eager = !graph && S.persistent_grid == 0;
+    int small[2];  // FP64 workgroups beside the matrix-core kernel still to be launched, by plane storage
+    for (int half = 0; half < 2; half++) small[half] = mfma ? 3 * P.ntiles_grp[map_group(1, half)] : 0;
     for (int cls = 0; cls < 2; cls++) {
         // on the matrix cores, class 0 also has the exact-split groups of float-input pairs
         const int nexact = (cls == 0 && mfma) ? 2 : 1;
         for (int exact = 0; exact < nexact; exact++)
             for (int half = 0; half < 2; half++) {
-                const int g = map_group(cls, half, exact);
                 if (half && !S.fp16) continue;
-                const int nsmall = cls == 0 && (P.ntiles_grp[g] > 0 || exact == 1) ? small[half] : 0;
-                if (!graph && P.ntiles_grp[g] == 0 && nsmall == 0) continue;
-                if (merged && cls == 1) continue;
-                // an eager launch of few tiles gives each channel of a tile its
-                // own workgroup (the same partials): fewer than two tiles per
-                // workgroup slot on the matrix-core kernel (4 per CU), and for
-                // the vector kernels (as few as 1 workgroup per CU in the FP64
-                // class) when the split workgroups fit in two rounds, as for
-                // one pair per call
-                const bool few = (cls == 0 && mfma) ? P.ntiles_grp[g] < 8 * S.num_cus
-                                                    : 3 * P.ntiles_grp[g] <= 2 * S.num_cus;
-                const int csplit = (!graph && S.persistent_grid == 0 && few) ? 3 : 1;
+                const int tiles = P.ntiles_grp[map_group(cls, half, exact)];
                 if (cls == 0 && mfma) {
-                    const int grid = P.ntiles_grp[g] > 0 || graph ? grid_for(P.ntiles_grp[g] * csplit, fixed) : 0;
-                    HIP_OR_THROW(launch_map_mx(half, exact, grid, nsmall, d.pairs, d.order_seg, d.order_start, d.hdr,
-                                               arena, partials, csplit, st),
+                    const MapSplit M = map_split(tiles, eager, S.num_cus);
+                    const int nsmall = eager && M.rows == 2 && tiles > 0 ? small[half] : 0;
+                    if (!graph && tiles == 0) continue;
+                    const int grid = grid_for(tiles * M.csplit, 2 * fixed, 2 * fixed);
+                    HIP_OR_THROW(launch_map_mx(half, exact, M.rows, grid, nsmall, d.pairs, d.order_seg, d.order_start,
+                                               d.hdr, arena, partials, M.csplit, st),
                                  E_BadDeviceCode);
                     small[half] -= nsmall;
                 } else if (mfma) {
-                    HIP_OR_THROW(launch_map_small(half, grid_for(3 * P.ntiles_grp[g], fixed), d.pairs, d.order_seg,
+                    if (!graph && small[half] == 0) continue;
+                    HIP_OR_THROW(launch_map_small(half, grid_for(small[half], fixed, fixed), d.pairs, d.order_seg,
                                                   d.order_start, d.hdr, arena, partials, st),
                                  E_BadDeviceCode);
                 } else {
-                    const int grid = grid_for(P.ntiles_grp[g] * csplit, cls == 0 ? fixed : std::max(1, fixed / 4));
+                    if (!graph && tiles == 0) continue;
+                    const int csplit = eager && 3 * tiles <= 2 * S.num_cus ? 3 : 1;
+                    const int grid = grid_for(tiles * csplit, fixed, cls == 0 ? fixed : std::max(1, fixed / 4));
                     HIP_OR_THROW(launch_map(half, cls, cls ? kSmallTH : S.map_th, grid, d.pairs, d.order_seg,
                                             d.order_start, d.hdr, arena, partials, taps, csplit, st),
                                  E_BadDeviceCode);

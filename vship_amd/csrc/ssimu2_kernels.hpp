@@ -18,12 +18,14 @@ hipError_t launch_map(bool half, int cls, int th, int grid, const PairDev* pairs
                       const Taps& taps, int csplit, hipStream_t st);
 // Map tiles of the FP32 class on the matrix cores (map_mfma.hip); exact: the
 // groups of float-input pairs (three-way bf16 split), else the scaled fp16
-// split. csplit: 1 (a workgroup per tile) or 3 (a workgroup per tile and
-// channel; the same partials). nsmall workgroups ahead of the grid's own take
-// the FP64 tiles of the same plane storage, one per tile and channel.
-hipError_t launch_map_mx(bool half, bool exact, int grid, int nsmall, const PairDev* pairs, const int32_t* order_seg,
-                         const int32_t* order_start, const BatchHdr* hdr, const void* arena, double* partials,
-                         int csplit, hipStream_t st);
+// split. rows: 1 (workgroups of two waves, each with all rows of 32 columns of
+// a tile) or 2 (four waves, each with half of the rows); csplit: 1 (a workgroup
+// per tile) or 3 (a workgroup per tile and channel); the same partials. With
+// rows 2, nsmall workgroups ahead of the grid's own take the FP64 tiles of the
+// same plane storage, one per tile and channel.
+hipError_t launch_map_mx(bool half, bool exact, int rows, int grid, int nsmall, const PairDev* pairs,
+                         const int32_t* order_seg, const int32_t* order_start, const BatchHdr* hdr, const void* arena,
+                         double* partials, int csplit, hipStream_t st);
 // The FP64 tiles beside the matrix-core kernel by themselves, walked by a grid
 // of any size.
 hipError_t launch_map_small(bool half, int grid, const PairDev* pairs, const int32_t* order_seg,
