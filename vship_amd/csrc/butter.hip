@@ -139,18 +139,19 @@ __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* 
     }
 }
 
-// 4:2:0 with left-located chroma: 64 x 64 luma tiles, the chroma
+// 4:2:0 with left-located chroma: kInputW x kInputH luma tiles, the chroma
 // neighbourhood staged in LDS (as the SSIMULACRA2 prep kernel does); a
 // thread converts four 2 x 2 quads per image.
+constexpr int kInputW = 128, kInputH = 32;
 template <bool WIDE>
 __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDesc* __restrict__ pairs, Scale S0,
                                                                    Scale S1, float scale) {
-    __shared__ float ch[2][kCh420][kCh420 + 1];
+    __shared__ float ch[2][kInputH / 2 + 4][kInputW / 2 + 3];
     const TileIdx ti = tile_of_block();
     const int pair = ti.z;
     const PairDesc& P = pairs[pair];
     const int W = S0.w, H = S0.h;
-    const int x0 = ti.x * 64, y0 = ti.y * 64;
+    const int x0 = ti.x * kInputW, y0 = ti.y * kInputH;
     const int maxcode = WIDE ? (1 << P.bits) - 1 : 255;
     const float sc = (float)(1 << (P.bits - 8));
     const float ymul = 1.0f / (219.0f * sc), yadd = -16.0f / 219.0f;
@@ -161,12 +162,12 @@ __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDes
         const uint8_t* const* src = P.src[im];
         const int64_t* stride = P.stride[im];
         __syncthreads();
-        stage_chroma420(ch, src, stride, W, H, x0, y0, WIDE, maxcode);
+        stage_chroma420<kInputW / 2, kInputH / 2>(&ch[0][0][0], src, stride, W, H, x0, y0, WIDE, maxcode);
         __syncthreads();
 #pragma unroll 1
         for (int i = 0; i < 4; i++) {
             const int q = threadIdx.x + kThreads * i;
-            const int qy = q >> 5, qx = q & 31;
+            const int qy = q / (kInputW / 2), qx = q % (kInputW / 2);
             const int xa = x0 + 2 * qx, ya = y0 + 2 * qy;
             if (xa >= W || ya >= H) continue;
             const bool hx = xa + 1 < W, hy = ya + 1 < H;
@@ -176,8 +177,8 @@ __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDes
                                  sample_u(src[0], stride[0], xb, ya, WIDE, maxcode),
                                  sample_u(src[0], stride[0], xb, yb, WIDE, maxcode)};
             float cb[4], cr[4];
-            chroma420_quad(ch[0], qx, qy, hx, hy, cmul, cadd, cb);
-            chroma420_quad(ch[1], qx, qy, hx, hy, cmul, cadd, cr);
+            chroma420_quad(&ch[0][0][0], kInputW / 2 + 3, qx, qy, hx, hy, cmul, cadd, cb);
+            chroma420_quad(&ch[1][0][0], kInputW / 2 + 3, qx, qy, hx, hy, cmul, cadd, cr);
             float lin[4][3];  // (xa,ya), (xa,yb), (xb,ya), (xb,yb)
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -1449,7 +1450,7 @@ void Engine::launch(int fmt, int n, bool general) {
     const dim3 gi(cdiv(w2_, 16), cdiv(h2_, 16), n);
     auto input = [&] {
         if (staged420_) {
-            const dim3 g4(cdiv(w_, 64), cdiv(h_, 64), n);
+            const dim3 g4(cdiv(w_, kInputW), cdiv(h_, kInputH), n);
             if (fmt == IN_YUV420_U16)
                 butter_input420_kernel<true><<<g4, dim3(kThreads), 0, stream_>>>(desc_d_, S0, S1, lin);
             else

@@ -105,7 +105,7 @@ PairLayout pair_layout(int w, int h, bool fp16) {
 
 int64_t pair_bytes(int w, int h, bool fp16) { return 2 * pair_layout(w, h, fp16).img_bytes; }
 
-int prep_tiles(int w, int h) { return 2 * ((w + kPrepTile - 1) / kPrepTile) * ((h + kPrepTile - 1) / kPrepTile); }
+int prep_tiles(int w, int h) { return 2 * ((w + kPrepW - 1) / kPrepW) * ((h + kPrepH - 1) / kPrepH); }
 
 int map_tiles(int w, int h, int th) {
     int n = 0, ww = w, hh = h;

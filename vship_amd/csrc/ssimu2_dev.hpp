@@ -15,7 +15,7 @@
 namespace vship {
 
 constexpr int kScales = 6;
-constexpr int kPrepTile = 64;   // scale-0 tile edge of the convert/pyramid kernel
+constexpr int kPrepW = 128, kPrepH = 32;  // scale-0 tile of the convert/pyramid kernel
 constexpr int kMapTW = 32;      // map tile width (columns)
 constexpr int kFeat = 18;       // partial sums per map tile: 3 channels x 3 maps x {sum d, sum d^4}
 constexpr int kHalfScales = 2;  // scales stored in FP16 when FP16 storage is on

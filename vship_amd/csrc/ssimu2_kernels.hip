@@ -72,17 +72,17 @@ __device__ __forceinline__ void to_xyb(float r, float g, float b, float& X, floa
 // prep kernel
 // ---------------------------------------------------------------------------
 struct PrepLds {
-    float l1[3][32][33];  // linear RGB of scales 1..4
+    float l1[3][kPrepH / 2][kPrepW / 2];  // linear RGB of scales 1..4
     // the staged chroma is read only while scales 0 and 1 are formed, the
-    // coarser levels only after: they share their memory, and the chroma rows
-    // carry no pad word, so that the struct is 23,040 bytes (45 blocks of
-    // 512) and seven workgroups fit in one CU's LDS
+    // coarser levels only after: they share their memory, and the rows carry
+    // no pad words, so that the struct is 23,008 bytes and seven workgroups
+    // fit in one CU's LDS
     union {
-        float ch[2][36][36];  // staged chroma neighbourhood of the tile (clamped indices)
+        float ch[2][kPrepH / 2 + 4][kPrepW / 2 + 3];  // staged chroma neighbourhood of the tile (clamped indices)
         struct {
-            float l2[3][16][17];
-            float l3[3][8][9];
-            float l4[3][4][5];
+            float l2[3][kPrepH / 4][kPrepW / 4 + 1];
+            float l3[3][kPrepH / 8][kPrepW / 8 + 1];
+            float l4[3][kPrepH / 16][kPrepW / 16 + 1];
         };
     };
 };
@@ -137,6 +137,21 @@ __device__ __forceinline__ void store_row4<__half>(uint8_t* arena, const PairDev
                                 reinterpret_cast<u2*>(b + o));
 }
 
+// Two pixels x, x + 1 (x even), in one 8-byte (FP16 planes: 4-byte) store.
+template <typename T>
+__device__ __forceinline__ void store_row2(uint8_t* arena, const PairDev& P, int img, int s, int c, int x, int y,
+                                           float v0, float v1) {
+    uint8_t* b = arena + P.arena_off + img * P.img_bytes + P.scale_off[s] + c * P.plane_elems[s] * (int64_t)sizeof(T);
+    const uint32_t o = ((uint32_t)y * (uint32_t)P.pitch[s] + (uint32_t)x) * (uint32_t)sizeof(T);
+    if constexpr (sizeof(T) == 4) {
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store((f2){v0, v1}, reinterpret_cast<f2*>(b + o));
+    } else {
+        const __half2 h = __floats2half2_rn(v0, v1);
+        __builtin_nontemporal_store(*reinterpret_cast<const uint32_t*>(&h), reinterpret_cast<uint32_t*>(b + o));
+    }
+}
+
 // XYB of one pixel of scale s into the arena: planes of type ST for the two
 // finest scales, FP32 for the rest.
 template <typename ST>
@@ -151,46 +166,81 @@ __device__ __forceinline__ void store_xyb(uint8_t* arena, const PairDev& P, int 
 // One pyramid level in LDS: child(cx, cy) = mean of the 2x2 parents with the
 // parent index clamped to the last valid row/column
 // (src/ssimu2/downsample.hpp:3-19, summation order kept).
-template <int TS, int PP, int CP, typename ST>
+template <int TW, int TH, int PP, int CP, typename ST>
 __device__ __forceinline__ void pyr_level(const float* par, float* chi, uint8_t* arena, const PairDev& P, int img, int s,
                                           int tx, int ty, int npx, int npy) {
-    const int x0 = tx * TS, y0 = ty * TS;
-    const int nvx = min(TS, P.sw[s] - x0), nvy = min(TS, P.sh[s] - y0);
-    for (int idx = tid_in_loop(); idx < TS * TS; idx += blockDim.x) {
-        const int cy = idx / TS, cx = idx - cy * TS;
+    const int x0 = tx * TW, y0 = ty * TH;
+    const int nvx = min(TW, P.sw[s] - x0), nvy = min(TH, P.sh[s] - y0);
+    for (int idx = tid_in_loop(); idx < TW * TH; idx += blockDim.x) {
+        const int cy = idx / TW, cx = idx - cy * TW;
         if (cx >= nvx || cy >= nvy) continue;
         const int px0 = 2 * cx, py0 = 2 * cy;
         const int px1 = min(2 * cx + 1, npx - 1), py1 = min(2 * cy + 1, npy - 1);
         float v[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const float* pc = par + c * (2 * TS) * PP;
+            const float* pc = par + c * (2 * TH) * PP;
             float a = pc[py0 * PP + px0];
             a += pc[py1 * PP + px0];
             a += pc[py0 * PP + px1];
             a += pc[py1 * PP + px1];
             v[c] = a * 0.25f;
-            if (chi) chi[(c * TS + cy) * CP + cx] = v[c];
+            if (chi) chi[(c * TH + cy) * CP + cx] = v[c];
         }
         store_xyb<ST>(arena, P, img, s, x0 + cx, y0 + cy, v[0], v[1], v[2]);
     }
 }
 
-// Reads sample x of row y of an input plane of RGB format FMT as float (a
-// 32-bit byte offset from the plane base: the host refuses planes of 4 GiB
-// or more).
+// Two neighbouring samples of a row in one load, of whatever alignment the
+// caller's planes have: the bytes as one word, and the two values.
+template <int BYTES>
+struct __attribute__((packed)) Samples2;
+template <>
+struct __attribute__((packed)) Samples2<1> {
+    uint16_t w;
+    template <int K>
+    __device__ __forceinline__ uint32_t code() const { return K ? (uint32_t)w >> 8 : (uint32_t)w & 0xffu; }
+};
+template <>
+struct __attribute__((packed)) Samples2<2> {
+    uint32_t w;
+    template <int K>
+    __device__ __forceinline__ uint32_t code() const { return K ? w >> 16 : w & 0xffffu; }
+};
+template <>
+struct __attribute__((packed)) Samples2<4> {
+    uint32_t w[2];
+    template <int K>
+    __device__ __forceinline__ uint32_t code() const { return w[K]; }
+};
+template <int BYTES>
+__device__ __forceinline__ Samples2<BYTES> load2(const uint8_t* plane, int64_t stride, int x, int y) {
+    typedef Samples2<BYTES> S;
+    const auto* p = as_global(reinterpret_cast<const S*>(plane + ((uint32_t)y * (uint32_t)stride + BYTES * (uint32_t)x)));
+    S s;
+    __builtin_memcpy(&s, p, sizeof(S));
+    return s;
+}
+template <int FMT>
+__device__ __forceinline__ float rgb_value(uint32_t code) {
+    if constexpr (FMT == IN_RGB_U8) return (float)code * (1.0f / 255.0f);
+    else if constexpr (FMT == IN_RGB_U16) return (float)code * (1.0f / 65535.0f);
+    else if constexpr (FMT == IN_RGB_F16) return __half2float(__ushort_as_half((unsigned short)code));
+    else return __uint_as_float(code);
+}
+
+// Sample x of row y of an input plane of RGB format FMT as float (a 32-bit byte
+// offset from the plane base: the host refuses planes of 4 GiB or more).
 template <int FMT>
 __device__ __forceinline__ float rgb_sample(const uint8_t* plane, int64_t stride, int x, int y) {
     constexpr uint32_t bps = FMT == IN_RGB_U8 ? 1 : (FMT == IN_RGB_F32 ? 4 : 2);
     const uint8_t* p = plane + ((uint32_t)y * (uint32_t)stride + bps * (uint32_t)x);
-    if constexpr (FMT == IN_RGB_U8) return (float)*as_global(p) * (1.0f / 255.0f);
-    else if constexpr (FMT == IN_RGB_U16) return (float)*as_global(reinterpret_cast<const uint16_t*>(p)) * (1.0f / 65535.0f);
-    else if constexpr (FMT == IN_RGB_F16)
-        return __half2float(__ushort_as_half(*as_global(reinterpret_cast<const unsigned short*>(p))));
-    else return *as_global(reinterpret_cast<const float*>(p));
+    if constexpr (bps == 1) return rgb_value<FMT>(*as_global(p));
+    else if constexpr (bps == 2) return rgb_value<FMT>(*as_global(reinterpret_cast<const uint16_t*>(p)));
+    else return rgb_value<FMT>(*as_global(reinterpret_cast<const uint32_t*>(p)));
 }
 
-// Scales 0 and 1 of one 64x64 tile of an image of input format FMT: a thread
+// Scales 0 and 1 of one tile of an image of input format FMT: a thread
 // owns 2x2 pixel quads of scale 0, so the scale-1 child is formed in
 // registers and also left in LDS (l1) for the coarser levels. For YUV, FMT is
 // IN_YUV420_U8 or IN_YUV420_U16 (the container), and GEN selects the generic
@@ -202,16 +252,27 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
     constexpr bool wide = FMT == IN_YUV420_U16;
     const int tid = tid_in_loop();
     const int W = P.w, H = P.h;
-    const int x0 = tx * kPrepTile, y0 = ty * kPrepTile;
+    const int x0 = tx * kPrepW, y0 = ty * kPrepH;
     const uint8_t* const* src = P.src[img];
     const int64_t* stride = P.stride[img];
     const int maxcode = wide ? (1 << P.bits) - 1 : 255;
+    // thread t takes the quads of column t % 64 in rows 4 (t / 64) .. +3; the
+    // staged 4:2:0 path keeps the horizontal chroma results of the eight staged
+    // rows these four quads read in registers, each row computed once
+    const int qx = tid & 63, qy0 = 4 * (tid >> 6);
+    constexpr int BPS = FMT == IN_RGB_U8 || (yuv && !wide) ? 1 : FMT == IN_RGB_F32 ? 4 : 2;
+    // whole quads of the staged path: all luma is under way before the chroma is staged
+    Samples2<BPS> luma[4][2];
+    if constexpr (FULL && yuv && !GEN) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) luma[i][k] = load2<BPS>(src[0], stride[0], x0 + 2 * qx, y0 + 2 * (qy0 + i) + k);
+    }
 
     if constexpr (yuv && !GEN) {
-        // stage the 36x36 chroma neighbourhood (indices clamped to the plane)
-        // thread t < 252 owns column t % 36 and rows t / 36 + 7k of both planes,
-        // so a wave reads whole row runs and the clamped column is computed once
-        stage_chroma420(L.ch, src, stride, W, H, x0, y0, wide, maxcode);
+        // stage the chroma neighbourhood (indices clamped to the plane)
+        stage_chroma420<kPrepW / 2, kPrepH / 2>(&L.ch[0][0][0], src, stride, W, H, x0, y0, wide, maxcode);
         __syncthreads();
     }
 
@@ -228,13 +289,8 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
     const float kr = P.kr, kb = P.kb, ikg = P.ikg;
     const float rcr = 2.0f * (1.0f - kr), bcb = 2.0f * (1.0f - kb);
 
-    const int nv1x = min(32, P.sw[1] - tx * 32), nv1y = min(32, P.sh[1] - ty * 32);
+    const int nv1x = min(kPrepW / 2, P.sw[1] - tx * (kPrepW / 2)), nv1y = min(kPrepH / 2, P.sh[1] - ty * (kPrepH / 2));
     constexpr bool full = FULL;
-    // thread t takes the quads of column t % 32 in rows 4 (t / 32) .. +3 (lanes
-    // 2k and 2k+1 still hold horizontally adjacent quads); the staged 4:2:0
-    // path keeps the horizontal chroma results of the eight staged rows these
-    // four quads read in registers, each row computed once
-    const int qx = tid & 31, qy0 = 4 * (tid >> 5);
     float che[2][8], cho[2][8];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -250,7 +306,16 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
         const bool hx = FULL || xa + 1 < W, hy = FULL || ya + 1 < H;
         const int xb = hx ? xa + 1 : xa, yb = hy ? ya + 1 : ya;  // clamped second column/row
         float rgb[4][3];  // quad pixels: (xa,ya), (xa,yb), (xb,ya), (xb,yb)
-        if constexpr (!yuv) {
+        if constexpr (!yuv && FULL) {
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const Samples2<BPS> v = load2<BPS>(src[p], stride[p], xa, ya + k);
+                    rgb[k][p] = rgb_value<FMT>(v.template code<0>());
+                    rgb[2 + k][p] = rgb_value<FMT>(v.template code<1>());
+                }
+        } else if constexpr (!yuv) {
 #pragma unroll
             for (int p = 0; p < 3; p++) {
                 rgb[0][p] = rgb_sample<FMT>(src[p], stride[p], xa, ya);
@@ -259,10 +324,20 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
                 rgb[3][p] = rgb_sample<FMT>(src[p], stride[p], xb, yb);
             }
         } else {
-            const float yv[4] = {sample_u(src[0], stride[0], xa, ya, wide, maxcode),
-                                 sample_u(src[0], stride[0], xa, yb, wide, maxcode),
-                                 sample_u(src[0], stride[0], xb, ya, wide, maxcode),
-                                 sample_u(src[0], stride[0], xb, yb, wide, maxcode)};
+            float yv[4];
+            if constexpr (FULL && !GEN) {
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const int a = (int)luma[i][k].template code<0>(), b = (int)luma[i][k].template code<1>();
+                    yv[k] = (float)(wide ? min(a, maxcode) : a);
+                    yv[2 + k] = (float)(wide ? min(b, maxcode) : b);
+                }
+            } else {
+                yv[0] = sample_u(src[0], stride[0], xa, ya, wide, maxcode);
+                yv[1] = sample_u(src[0], stride[0], xa, yb, wide, maxcode);
+                yv[2] = sample_u(src[0], stride[0], xb, ya, wide, maxcode);
+                yv[3] = sample_u(src[0], stride[0], xb, yb, wide, maxcode);
+            }
             float cbcr[2][4];
             if constexpr (GEN) {
                 const int csw = P.csw, csh = P.csh;
@@ -297,21 +372,16 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
 #pragma unroll
             for (int p = 0; p < 3; p++) rgb[k][p] = linearize(rgb[k][p]);
         if (full) {
-            // every lane of the wave is here (no quad of a full tile is out of
-            // the image); lanes 2k and 2k+1 hold horizontally adjacent quads:
-            // the even lane writes both quads' first row, the odd lane their
-            // second row, four consecutive pixels per plane in one store
+            // a wave writes whole rows of the tile: 64 lanes, two pixels each
+            // (lanes that exchanged two of their four pixels, to write 16
+            // bytes each, spent 6 % of the kernel's vector issue on it)
             float v[3][4];
 #pragma unroll
             for (int k = 0; k < 4; k++) to_xyb(rgb[k][0], rgb[k][1], rgb[k][2], v[0][k], v[1][k], v[2][k]);
-            const bool odd = qx & 1;
-            const int sx = odd ? xa - 2 : xa, sy = odd ? yb : ya;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                const float s0 = odd ? v[c][0] : v[c][1], s1 = odd ? v[c][2] : v[c][3];
-                const float r0 = __shfl_xor(s0, 1, 64), r1 = __shfl_xor(s1, 1, 64);
-                const float4 o = odd ? make_float4(r0, r1, v[c][1], v[c][3]) : make_float4(v[c][0], v[c][2], r0, r1);
-                store_row4<ST>(arena, P, img, 0, c, sx, sy, o);
+                store_row2<ST>(arena, P, img, 0, c, xa, ya, v[c][0], v[c][2]);
+                store_row2<ST>(arena, P, img, 0, c, xa, yb, v[c][1], v[c][3]);
             }
         } else {
             store_xyb<ST>(arena, P, img, 0, xa, ya, rgb[0][0], rgb[0][1], rgb[0][2]);
@@ -338,23 +408,23 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
 // is complete (no clamps, no selects of the chroma filter outputs).
 template <typename ST, int FMT, bool GEN = false>
 __device__ __forceinline__ void prep_quads(PrepLds& L, const PairDev& P, uint8_t* arena, int img, int tx, int ty) {
-    if ((tx + 1) * kPrepTile <= P.w && (ty + 1) * kPrepTile <= P.h)
+    if ((tx + 1) * kPrepW <= P.w && (ty + 1) * kPrepH <= P.h)
         prep_quads_body<ST, FMT, GEN, true>(L, P, arena, img, tx, ty);
     else
         prep_quads_body<ST, FMT, GEN, false>(L, P, arena, img, tx, ty);
 }
 
-// XYB of the tile's 32x32 scale-1 pixels from their linear RGB in LDS: thread
-// t takes pixels 4 (t % 8) .. +3 of row t / 8, one 16-byte store per plane for
-// four whole pixels (a wave writes eight 128-byte rows per plane), pixel by
+// XYB of the tile's 64x16 scale-1 pixels from their linear RGB in LDS: thread
+// t takes pixels 4 (t % 16) .. +3 of row t / 16, one 16-byte store per plane for
+// four whole pixels (a wave writes four 256-byte rows per plane), pixel by
 // pixel where the row ends inside the four.
 template <typename ST>
 __device__ __forceinline__ void store_scale1(const PrepLds& L, const PairDev& P, uint8_t* arena, int img, int tx,
                                              int ty, int nv1x, int nv1y) {
     const int tid = tid_in_loop();
-    const int r = tid >> 3, c4 = (tid & 7) * 4;
+    const int r = tid >> 4, c4 = (tid & 15) * 4;
     if (r >= nv1y || c4 >= nv1x) return;
-    const int x = tx * 32 + c4, y = ty * 32 + r;
+    const int x = tx * (kPrepW / 2) + c4, y = ty * (kPrepH / 2) + r;
     if (c4 + 4 <= nv1x) {
         float v[3][4];
 #pragma unroll
@@ -367,16 +437,24 @@ __device__ __forceinline__ void store_scale1(const PrepLds& L, const PairDev& P,
     }
 }
 
-// Each workgroup converts one 64x64 scale-0 tile of one image. Scales 0 and 1
+// Each workgroup converts one scale-0 tile of one image. Scales 0 and 1
 // come from prep_quads, instantiated per input format; scales 2..5 go through
 // LDS. Every XYB plane is written exactly once. GEN = false takes the RGB and
 // staged 4:2:0 pairs, GEN = true the pairs of the generic chroma path; each
 // skips the other's tiles. Both are held to seven waves per SIMD (at most 72
 // VGPRs, no spills: the thread-index arithmetic is recomputed per use rather
 // than held across the tile loop, see tid_in_loop), which overlaps one
-// tile's stores with another's arithmetic: at 1920x1080 (240 pairs) the
-// kernel took 3.95 ms at seven waves per SIMD, 4.24 ms at six and 4.38 ms at
-// five, before the full-tile loop took it to 3.78 ms.
+// tile's stores with another's arithmetic.
+//
+// What bounds it is its writes (66 MB per 1080p pair, at 4.7 of the 5.6 TB/s a
+// write-only loop reaches), then vector issue. Tiles of 128 x 32 read half as
+// many lines twice as tiles of 64 x 64 (96 1080p pairs 0.98 -> 0.60 million
+// counted reads), a wave's lanes are one row of them, and a tile's samples are
+// loaded together, luma before the chroma is staged: one pair after another, as
+// the staging loop had it, the wider tiles were 4 % slower. 240 1080p pairs, the
+// whole batch: 11.02 -> 10.66 ms; 24 pairs of RGB u8, u16, f16, f32: 1,128,
+// 1,207, 1,464, 1,579 -> 1,077, 1,127, 1,381, 1,498 us; 24 4K 10-bit pairs
+// with FP16 planes 3.67 -> 3.58 ms.
 template <typename ST, bool GEN>
 __global__ __launch_bounds__(256, 7) void prep_kernel(const PairDev* __restrict__ pairs,
                                                    const int32_t* __restrict__ prep_start,
@@ -394,7 +472,7 @@ __global__ __launch_bounds__(256, 7) void prep_kernel(const PairDev* __restrict_
         }
         const PairDev& P = pairs[lo];
         const int W = P.w, H = P.h;
-        const int ntx = (W + kPrepTile - 1) / kPrepTile, nty = (H + kPrepTile - 1) / kPrepTile;
+        const int ntx = (W + kPrepW - 1) / kPrepW, nty = (H + kPrepH - 1) / kPrepH;
         int local = t - prep_start[lo];
         const int img = local / (ntx * nty);
         local -= img * ntx * nty;
@@ -417,20 +495,29 @@ __global__ __launch_bounds__(256, 7) void prep_kernel(const PairDev* __restrict_
             }
         }
         __syncthreads();
-        const int nv1x = min(32, P.sw[1] - tx * 32), nv1y = min(32, P.sh[1] - ty * 32);
-        store_scale1<ST>(L, P, arena, img, tx, ty, nv1x, nv1y);
+        auto valid = [&](int sc, int& nx, int& ny) {  // the tile's part of scale sc that lies in the image
+            nx = min(kPrepW >> sc, P.sw[sc] - tx * (kPrepW >> sc));
+            ny = min(kPrepH >> sc, P.sh[sc] - ty * (kPrepH >> sc));
+        };
+        int nx, ny;
+        valid(1, nx, ny);
+        store_scale1<ST>(L, P, arena, img, tx, ty, nx, ny);
 
         // scales 2..5 from LDS
-        pyr_level<16, 33, 17, ST>(&L.l1[0][0][0], &L.l2[0][0][0], arena, P, img, 2, tx, ty, nv1x, nv1y);
+        pyr_level<kPrepW / 4, kPrepH / 4, kPrepW / 2, kPrepW / 4 + 1, ST>(&L.l1[0][0][0], &L.l2[0][0][0], arena, P, img,
+                                                                          2, tx, ty, nx, ny);
         __syncthreads();
-        const int nv2x = min(16, P.sw[2] - tx * 16), nv2y = min(16, P.sh[2] - ty * 16);
-        pyr_level<8, 17, 9, ST>(&L.l2[0][0][0], &L.l3[0][0][0], arena, P, img, 3, tx, ty, nv2x, nv2y);
+        valid(2, nx, ny);
+        pyr_level<kPrepW / 8, kPrepH / 8, kPrepW / 4 + 1, kPrepW / 8 + 1, ST>(&L.l2[0][0][0], &L.l3[0][0][0], arena, P,
+                                                                              img, 3, tx, ty, nx, ny);
         __syncthreads();
-        const int nv3x = min(8, P.sw[3] - tx * 8), nv3y = min(8, P.sh[3] - ty * 8);
-        pyr_level<4, 9, 5, ST>(&L.l3[0][0][0], &L.l4[0][0][0], arena, P, img, 4, tx, ty, nv3x, nv3y);
+        valid(3, nx, ny);
+        pyr_level<kPrepW / 16, kPrepH / 16, kPrepW / 8 + 1, kPrepW / 16 + 1, ST>(&L.l3[0][0][0], &L.l4[0][0][0], arena,
+                                                                                 P, img, 4, tx, ty, nx, ny);
         __syncthreads();
-        const int nv4x = min(4, P.sw[4] - tx * 4), nv4y = min(4, P.sh[4] - ty * 4);
-        pyr_level<2, 5, 1, ST>(&L.l4[0][0][0], (float*)nullptr, arena, P, img, 5, tx, ty, nv4x, nv4y);
+        valid(4, nx, ny);
+        pyr_level<kPrepW / 32, kPrepH / 32, kPrepW / 16 + 1, 1, ST>(&L.l4[0][0][0], (float*)nullptr, arena, P, img, 5, tx,
+                                                                    ty, nx, ny);
         __syncthreads();
     }
 }

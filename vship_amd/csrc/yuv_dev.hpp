@@ -84,30 +84,39 @@ __device__ __forceinline__ float chroma_at(const uint8_t* plane, int64_t stride,
     return a;
 }
 
-// 4:2:0 with left-located chroma (the common case), staged: the 36 x 36
-// chroma neighbourhood of a 64 x 64 luma tile at (x0, y0), origin
-// (x0 / 2 - 1, y0 / 2 - 2), indices clamped to the plane. Thread t < 252 owns
-// column t % 36 and rows t / 36 + 7 k of both planes, so a wave reads whole
-// row runs and the clamped column is computed once. PITCH: floats per staged
-// row (36, or 37 with a pad word).
-constexpr int kCh420 = 36;
-
-template <int PITCH>
-__device__ __forceinline__ void stage_chroma420(float (*ch)[kCh420][PITCH], const uint8_t* const* src,
-                                                const int64_t* stride, int W, int H, int x0, int y0, bool wide,
-                                                int maxcode) {
+// 4:2:0 with left-located chroma (the common case), staged: the neighbourhood
+// of QW + 3 columns and QH + 4 rows of both planes of a tile of QW x QH quads
+// at luma (x0, y0), origin (x0 / 2 - 1, y0 / 2 - 2), indices clamped to the
+// plane, into rows of QW + 3 floats. A wave reads whole row runs of 64 columns;
+// the columns beyond come last.
+template <int QW, int QH>
+__device__ __forceinline__ void stage_chroma420(float* ch, const uint8_t* const* src, const int64_t* stride, int W,
+                                                int H, int x0, int y0, bool wide, int maxcode) {
+    constexpr int NC = QW + 3, NR = QH + 4, MAIN = 64, REST = NC - MAIN;
+    static_assert(QW == MAIN, "a wave's lanes take a row of the tile's quads");
     const int tid = tid_in_loop();
     const int cw = (W + 1) >> 1, chh = (H + 1) >> 1;
     const int cx0 = x0 / 2 - 1, cy0 = y0 / 2 - 2;
-    if (tid < 252) {
-        const int c = tid % 36;
-        const int gx = min(max(cx0 + c, 0), cw - 1);
-        for (int r = tid / 36; r < 36; r += 7) {
-            const int gy = min(max(cy0 + r, 0), chh - 1);
-            ch[0][r][c] = sample_u(src[1], stride[1], gx, gy, wide, maxcode);
-            ch[1][r][c] = sample_u(src[2], stride[2], gx, gy, wide, maxcode);
-        }
+    static_assert(NR % 4 == 0 && 2 * NR * REST <= 256, "the same work for each wave, a thread for each sample beyond");
+    // all of a thread's loads before its first store
+    const int c = tid & 63, r0 = tid >> 6, gx = min(max(cx0 + c, 0), cw - 1);
+    float v[2][NR / 4], beyond = 0.f;
+#pragma unroll
+    for (int k = 0; k < NR / 4; k++) {
+        const int gy = min(max(cy0 + r0 + 4 * k, 0), chh - 1);
+        v[0][k] = sample_u(src[1], stride[1], gx, gy, wide, maxcode);
+        v[1][k] = sample_u(src[2], stride[2], gx, gy, wide, maxcode);
     }
+    const int bc = MAIN + tid % REST, br = tid / REST;  // row br % NR of plane br / NR
+    const int bgx = min(max(cx0 + bc, 0), cw - 1), bgy = min(max(cy0 + br % NR, 0), chh - 1);
+    if (tid < NR * REST) beyond = sample_u(src[1], stride[1], bgx, bgy, wide, maxcode);
+    else if (tid < 2 * NR * REST) beyond = sample_u(src[2], stride[2], bgx, bgy, wide, maxcode);
+#pragma unroll
+    for (int k = 0; k < NR / 4; k++) {
+        ch[(r0 + 4 * k) * NC + c] = v[0][k];
+        ch[(NR + r0 + 4 * k) * NC + c] = v[1][k];
+    }
+    if (tid < 2 * NR * REST) ch[br * NC + bc] = beyond;
 }
 
 // Chroma (scaled by cmul, offset by cadd) of the quad of luma pixels
@@ -140,11 +149,11 @@ __device__ __forceinline__ void chroma420_vquad(const float* he, const float* ho
 }
 
 // Both steps for one quad, the five rows filtered here.
-__device__ __forceinline__ void chroma420_quad(const float (*ch)[kCh420 + 1], int qx, int qy, bool hx, bool hy,
+__device__ __forceinline__ void chroma420_quad(const float* ch, int pitch, int qx, int qy, bool hx, bool hy,
                                                float cmul, float cadd, float out[4]) {
     float he[5], ho[5];
 #pragma unroll
-    for (int r = 0; r < 5; r++) chroma420_hrow(ch[qy + r], qx, he[r], ho[r]);
+    for (int r = 0; r < 5; r++) chroma420_hrow(ch + (qy + r) * pitch, qx, he[r], ho[r]);
     chroma420_vquad(he, ho, hx, hy, cmul, cadd, out);
 }
 
