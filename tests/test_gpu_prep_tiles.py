@@ -67,3 +67,27 @@ def test_tiles_and_alignment(w, h, fmt, bits):
         s, f = b.compute(desc, features=True)
     buf.free()
     assert s[0] == got and np.array_equal(f, feats)
+
+
+@pytest.mark.parametrize("layout,bits,loc", [("444", 8, api.CHROMA_LEFT), ("444", 10, api.CHROMA_CENTER),
+                                             ("422", 8, api.CHROMA_LEFT), ("422", 10, api.CHROMA_TOPLEFT),
+                                             ("422", 16, api.CHROMA_LEFT), ("422", 8, api.CHROMA_CENTER)])
+@pytest.mark.parametrize("w,h", [(257, 32), (384, 64), (387, 65), (518, 97)])
+def test_layouts_of_whole_tiles(w, h, layout, bits, loc):
+    """Whole tiles of 4:4:4 and left-located 4:2:2 load their chroma directly; the tiles at the picture's sides,
+    and every other layout, form each sample's position and weights."""
+    f8, f16, sw, sh = api.YUV_LAYOUTS[layout]
+    say(f"case prep layouts {w}x{h} YUV{layout} {bits}-bit location {loc}")
+    rng = np.random.default_rng(w + h + bits)
+    s, dt = 1 << (bits - 8), np.uint8 if bits == 8 else np.uint16
+    f, _ = rgb_pair(w, h, api.PF_RGB_F32, w + bits)
+    sub = (slice(None, None, 1 << sh), slice(None, None, 1 << sw))
+    ref = [np.round(16 * s + r * s * p.astype(np.float64)).astype(dt)
+           for r, p in ((219, f[0]), (224, f[1][sub]), (224, f[2][sub]))]
+    # (codes beyond a 10-bit depth are clamped to it)
+    dist = [np.clip(np.round(p + 3 * s * rng.standard_normal(p.shape)), 0, (1 << bits) - 1 + (bits == 10) * 3).astype(dt)
+            for p in ref]
+    want, fo = ol.score_yuv(ref, dist, bits, ol.SO_MAT_BT709, sw, sh, loc)
+    (got,), feats = gpu_batch([(ref, dist)], f8 if bits == 8 else f16, bits=bits, chroma_location=loc)
+    assert abs(got - want) <= SCORE_ATOL
+    assert np.all(np.abs(feats[0] - fo) <= 2e-5 + 1e-3 * np.abs(fo))
