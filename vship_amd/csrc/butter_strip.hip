@@ -67,13 +67,15 @@ constexpr float kXybMax = 8192.0f;
 // 16 b on and then, if kStep2 is not 0, the next kStep2; a single block reads
 // the first kCols - 16 columns from its own kCol0 on. Of the column pass the
 // ring holds kRing blocks of 16 rows, the first kRowOff rows above the output
-// block. LDS rows of kPitch bytes put the 16-byte operand reads of 16 lanes in
-// distinct banks.
+// block. LDS rows of kPitch bytes put the 16-byte operand reads of 8 or 16 lanes
+// in distinct banks; at 96, without a pad, four opsin workgroups fit in a CU's
+// LDS (three took 0.57 ms for sixteen 1080p pairs, four 0.54), with fewer
+// conflicts than at 112.
 template <int R>
 struct Geo;
 template <>
 struct Geo<8> {  // 16 + 2 * 8 = 32 columns and rows
-    static constexpr int kCol0 = -8, kCols = 48, kPitch = 112, kStep2 = 0, kRing = 2, kRowOff = 8;
+    static constexpr int kCol0 = -8, kCols = 48, kPitch = 96, kStep2 = 0, kRing = 2, kRowOff = 8;
 };
 template <>
 struct Geo<9> {  // 34 columns and rows
@@ -226,7 +228,7 @@ __device__ __forceinline__ void load_centres(Centres<P>& C, const Scale& S, int 
 // both images, and the difference of the two Bs, all that the later stages
 // need of it (they are linear in B)
 struct OpsinStage {
-    static constexpr int R = 8, kSig = SG_OPSIN, kPlanes = 6, kSrc = Q_LIN, kCentres = 6, kWaves = 3;
+    static constexpr int R = 8, kSig = SG_OPSIN, kPlanes = 6, kSrc = Q_LIN, kCentres = 6, kWaves = 4;
     template <bool NT>
     static __device__ __forceinline__ void points(const Exchange<6>& E, const Px& X, const Centres<6>& C,
                                                   const Scale& S, int pair, const StripArgs& A) {
@@ -332,7 +334,7 @@ struct MidStage {
 // differences, L2 terms and mask inputs (separatefrequencies.hpp:117-140,
 // 190-200; simplerdiff.hpp:60-101; maskPsycho.hpp:24-40)
 struct HighStage {
-    static constexpr int R = 8, kSig = SG_HIGH, kPlanes = 4, kSrc = Q_HFR, kCentres = 4, kWaves = 3;
+    static constexpr int R = 8, kSig = SG_HIGH, kPlanes = 4, kSrc = Q_HFR, kCentres = 4, kWaves = 4;
     template <bool NT>
     static __device__ __forceinline__ void points(const Exchange<4>& E, const Px& X, const Centres<4>& C,
                                                   const Scale& S, int pair, const StripArgs& A) {
