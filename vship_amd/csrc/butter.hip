@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDes
         const uint8_t* const* src = P.src[im];
         const int64_t* stride = P.stride[im];
         __syncthreads();
-        stage_chroma420<kInputW / 2, kInputH / 2>(&ch[0][0][0], src, stride, W, H, x0, y0, WIDE, maxcode);
+        stage_chroma420<kInputW / 2, kInputH / 2, kThreads / 64>(&ch[0][0][0], src, stride, W, H, x0, y0, WIDE, maxcode);
         __syncthreads();
 #pragma unroll 1
         for (int i = 0; i < 4; i++) {

@@ -268,7 +268,7 @@ __device__ __forceinline__ float rgb_sample(const uint8_t* plane, int64_t stride
 // (With a position, weights and up to 16 loads per pixel and plane, eight 1080p
 // 4:2:2 10-bit pairs took 493 us, now 444; 24 4:4:4 8-bit ones 1,277, now 1,090.)
 enum Chroma { CH_ANY, CH_444, CH_422 };
-template <typename ST, int FMT, bool GEN, bool FULL, Chroma CH = CH_ANY>
+template <typename ST, int FMT, bool GEN, bool FULL, int QPT, Chroma CH = CH_ANY>
 __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, uint8_t* arena, int img, int tx, int ty) {
     constexpr bool yuv = FMT >= IN_YUV420_U8;
     constexpr bool wide = FMT == IN_YUV420_U16;
@@ -278,23 +278,23 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
     const uint8_t* const* src = P.src[img];
     const int64_t* stride = P.stride[img];
     const int maxcode = wide ? (1 << P.bits) - 1 : 255;
-    // thread t takes the quads of column t % 64 in rows 4 (t / 64) .. +3; the
-    // staged 4:2:0 path keeps the horizontal chroma results of the eight staged
-    // rows these four quads read in registers, each row computed once
-    const int qx = tid & 63, qy0 = 4 * (tid >> 6);
+    // thread t takes the quads of column t % 64 in rows QPT (t / 64) .. + QPT - 1;
+    // the staged 4:2:0 path keeps the horizontal chroma results of the QPT + 4
+    // staged rows these quads read in registers, each row computed once
+    const int qx = tid & 63, qy0 = QPT * (tid >> 6);
     constexpr int BPS = FMT == IN_RGB_U8 || (yuv && !wide) ? 1 : FMT == IN_RGB_F32 ? 4 : 2;
     // whole quads of the staged path: all luma is under way before the chroma is staged
-    Samples2<BPS> luma[4][2];
+    Samples2<BPS> luma[QPT][2];
     if constexpr (FULL && yuv && !GEN) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < QPT; i++)
 #pragma unroll
             for (int k = 0; k < 2; k++) luma[i][k] = load2<BPS>(src[0], stride[0], x0 + 2 * qx, y0 + 2 * (qy0 + i) + k);
     }
 
     if constexpr (yuv && !GEN) {
         // stage the chroma neighbourhood (indices clamped to the plane)
-        stage_chroma420<kPrepW / 2, kPrepH / 2>(&L.ch[0][0][0], src, stride, W, H, x0, y0, wide, maxcode);
+        stage_chroma420<kPrepW / 2, kPrepH / 2, kPrepH / 2 / QPT>(&L.ch[0][0][0], src, stride, W, H, x0, y0, wide, maxcode);
         __syncthreads();
     }
 
@@ -313,9 +313,9 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
 
     const int nv1x = min(kPrepW / 2, P.sw[1] - tx * (kPrepW / 2)), nv1y = min(kPrepH / 2, P.sh[1] - ty * (kPrepH / 2));
     constexpr bool full = FULL;
-    float che[2][8], cho[2][8];
+    float che[2][QPT + 4], cho[2][QPT + 4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < QPT; i++) {
         const int qy = qy0 + i;
         if constexpr (yuv && !GEN) {
 #pragma unroll
@@ -464,23 +464,23 @@ __device__ __forceinline__ void prep_quads_body(PrepLds& L, const PairDev& P, ui
 
 // A tile wholly inside the image takes an instantiation in which every quad
 // is complete (no clamps, no selects of the chroma filter outputs).
-template <typename ST, int FMT, bool GEN = false>
+template <typename ST, int QPT, int FMT, bool GEN = false>
 __device__ __forceinline__ void prep_quads(PrepLds& L, const PairDev& P, uint8_t* arena, int img, int tx, int ty) {
     if ((tx + 1) * kPrepW <= P.w && (ty + 1) * kPrepH <= P.h) {
         if constexpr (GEN) {
             // columns x0 / 2 - 1 .. x0 / 2 + kPrepW / 2 + 1 of a chroma plane of (w + 1) / 2
             if (P.csw == 0 && P.csh == 0)
-                prep_quads_body<ST, FMT, GEN, true, CH_444>(L, P, arena, img, tx, ty);
+                prep_quads_body<ST, FMT, GEN, true, QPT, CH_444>(L, P, arena, img, tx, ty);
             else if (P.csw == 1 && P.csh == 0 && !cloc_hcentred(P.cloc) && tx > 0 &&
                      (tx + 1) * (kPrepW / 2) + 2 <= (P.w + 1) / 2)
-                prep_quads_body<ST, FMT, GEN, true, CH_422>(L, P, arena, img, tx, ty);
+                prep_quads_body<ST, FMT, GEN, true, QPT, CH_422>(L, P, arena, img, tx, ty);
             else
-                prep_quads_body<ST, FMT, GEN, true>(L, P, arena, img, tx, ty);
+                prep_quads_body<ST, FMT, GEN, true, QPT>(L, P, arena, img, tx, ty);
         } else {
-            prep_quads_body<ST, FMT, GEN, true>(L, P, arena, img, tx, ty);
+            prep_quads_body<ST, FMT, GEN, true, QPT>(L, P, arena, img, tx, ty);
         }
     } else
-        prep_quads_body<ST, FMT, GEN, false>(L, P, arena, img, tx, ty);
+        prep_quads_body<ST, FMT, GEN, false, QPT>(L, P, arena, img, tx, ty);
 }
 
 // XYB of the tile's 64x16 scale-1 pixels from their linear RGB in LDS: thread
@@ -524,8 +524,11 @@ __device__ __forceinline__ void store_scale1(const PrepLds& L, const PairDev& P,
 // whole batch: 11.02 -> 10.66 ms; 24 pairs of RGB u8, u16, f16, f32: 1,128,
 // 1,207, 1,464, 1,579 -> 1,077, 1,127, 1,381, 1,498 us; 24 4K 10-bit pairs
 // with FP16 planes 3.67 -> 3.58 ms.
-template <typename ST, bool GEN>
-__global__ __launch_bounds__(256, 7) void prep_kernel(const PairDev* __restrict__ pairs,
+//
+// QPT: quads per thread, 4 in workgroups of 256 threads; 1 in workgroups of 1,024,
+// for launches of no more tiles than CUs, whose time is one tile's latency.
+template <typename ST, bool GEN, int QPT>
+__global__ __launch_bounds__(1024 / QPT, QPT == 4 ? 7 : 4) void prep_kernel(const PairDev* __restrict__ pairs,
                                                    const int32_t* __restrict__ prep_start,
                                                    const BatchHdr* __restrict__ hdr, uint8_t* __restrict__ arena) {
     __shared__ PrepLds L;
@@ -549,17 +552,17 @@ __global__ __launch_bounds__(256, 7) void prep_kernel(const PairDev* __restrict_
         if (prep_generic(P.fmt, P.csw, P.csh, P.cloc) != GEN) continue;  // uniform over the workgroup
 
         if constexpr (GEN) {
-            if (fmt_wide(P.fmt)) prep_quads<ST, IN_YUV420_U16, true>(L, P, arena, img, tx, ty);
-            else prep_quads<ST, IN_YUV420_U8, true>(L, P, arena, img, tx, ty);
+            if (fmt_wide(P.fmt)) prep_quads<ST, QPT, IN_YUV420_U16, true>(L, P, arena, img, tx, ty);
+            else prep_quads<ST, QPT, IN_YUV420_U8, true>(L, P, arena, img, tx, ty);
         } else {
             switch (P.fmt) {
-            case IN_RGB_U8: prep_quads<ST, IN_RGB_U8>(L, P, arena, img, tx, ty); break;
-            case IN_RGB_U16: prep_quads<ST, IN_RGB_U16>(L, P, arena, img, tx, ty); break;
-            case IN_RGB_F16: prep_quads<ST, IN_RGB_F16>(L, P, arena, img, tx, ty); break;
-            case IN_RGB_F32: prep_quads<ST, IN_RGB_F32>(L, P, arena, img, tx, ty); break;
+            case IN_RGB_U8: prep_quads<ST, QPT, IN_RGB_U8>(L, P, arena, img, tx, ty); break;
+            case IN_RGB_U16: prep_quads<ST, QPT, IN_RGB_U16>(L, P, arena, img, tx, ty); break;
+            case IN_RGB_F16: prep_quads<ST, QPT, IN_RGB_F16>(L, P, arena, img, tx, ty); break;
+            case IN_RGB_F32: prep_quads<ST, QPT, IN_RGB_F32>(L, P, arena, img, tx, ty); break;
             default:  // YUV 4:2:0 with left-located chroma: the staged path
-                if (fmt_wide(P.fmt)) prep_quads<ST, IN_YUV420_U16>(L, P, arena, img, tx, ty);
-                else prep_quads<ST, IN_YUV420_U8>(L, P, arena, img, tx, ty);
+                if (fmt_wide(P.fmt)) prep_quads<ST, QPT, IN_YUV420_U16>(L, P, arena, img, tx, ty);
+                else prep_quads<ST, QPT, IN_YUV420_U8>(L, P, arena, img, tx, ty);
                 break;
             }
         }
@@ -1019,16 +1022,20 @@ __global__ __launch_bounds__(kFinThreads) void finalize_kernel(const PairDev* __
 // ---------------------------------------------------------------------------
 // host-side launchers
 // ---------------------------------------------------------------------------
-hipError_t launch_prep(bool fp16, bool generic, int grid, const PairDev* pairs, const int32_t* prep_start,
+template <typename ST>
+static void launch_prep_t(bool generic, bool few, int grid, const PairDev* pairs, const int32_t* prep_start,
+                          const BatchHdr* hdr, uint8_t* arena, hipStream_t st) {
+    if (generic && few) prep_kernel<ST, true, 1><<<grid, 1024, 0, st>>>(pairs, prep_start, hdr, arena);
+    else if (generic) prep_kernel<ST, true, 4><<<grid, 256, 0, st>>>(pairs, prep_start, hdr, arena);
+    else if (few) prep_kernel<ST, false, 1><<<grid, 1024, 0, st>>>(pairs, prep_start, hdr, arena);
+    else prep_kernel<ST, false, 4><<<grid, 256, 0, st>>>(pairs, prep_start, hdr, arena);
+}
+
+hipError_t launch_prep(bool fp16, bool generic, bool few, int grid, const PairDev* pairs, const int32_t* prep_start,
                        const BatchHdr* hdr, void* arena, hipStream_t st) {
     uint8_t* a = reinterpret_cast<uint8_t*>(arena);
-    if (fp16) {
-        if (generic) prep_kernel<__half, true><<<grid, 256, 0, st>>>(pairs, prep_start, hdr, a);
-        else prep_kernel<__half, false><<<grid, 256, 0, st>>>(pairs, prep_start, hdr, a);
-    } else {
-        if (generic) prep_kernel<float, true><<<grid, 256, 0, st>>>(pairs, prep_start, hdr, a);
-        else prep_kernel<float, false><<<grid, 256, 0, st>>>(pairs, prep_start, hdr, a);
-    }
+    if (fp16) launch_prep_t<__half>(generic, few, grid, pairs, prep_start, hdr, a, st);
+    else launch_prep_t<float>(generic, few, grid, pairs, prep_start, hdr, a, st);
     return hipGetLastError();
 }
 

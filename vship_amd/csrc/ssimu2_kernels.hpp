@@ -7,8 +7,9 @@
 namespace vship {
 
 // generic: the prep kernel of the pairs on the generic chroma path
-// (prep_generic), else the one of every other pair.
-hipError_t launch_prep(bool fp16, bool generic, int grid, const PairDev* pairs, const int32_t* prep_start,
+// (prep_generic), else the one of every other pair. few: workgroups of 1,024
+// threads, for few tiles.
+hipError_t launch_prep(bool fp16, bool generic, bool few, int grid, const PairDev* pairs, const int32_t* prep_start,
                        const BatchHdr* hdr, void* arena, hipStream_t st);
 // Map tiles of one group: cls 0 FP32 moments with tile height th (48, 64 or
 // 112), cls 1 FP64 moments with tile height kSmallTH; half: the group's

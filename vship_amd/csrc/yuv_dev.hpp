@@ -87,9 +87,9 @@ __device__ __forceinline__ float chroma_at(const uint8_t* plane, int64_t stride,
 // 4:2:0 with left-located chroma (the common case), staged: the neighbourhood
 // of QW + 3 columns and QH + 4 rows of both planes of a tile of QW x QH quads
 // at luma (x0, y0), origin (x0 / 2 - 1, y0 / 2 - 2), indices clamped to the
-// plane, into rows of QW + 3 floats. A wave reads whole row runs of 64 columns;
-// the columns beyond come last.
-template <int QW, int QH>
+// plane, into rows of QW + 3 floats, by NW waves. A wave reads whole row runs of
+// 64 columns; the columns beyond come last.
+template <int QW, int QH, int NW>
 __device__ __forceinline__ void stage_chroma420(float* ch, const uint8_t* const* src, const int64_t* stride, int W,
                                                 int H, int x0, int y0, bool wide, int maxcode) {
     constexpr int NC = QW + 3, NR = QH + 4, MAIN = 64, REST = NC - MAIN;
@@ -97,13 +97,14 @@ __device__ __forceinline__ void stage_chroma420(float* ch, const uint8_t* const*
     const int tid = tid_in_loop();
     const int cw = (W + 1) >> 1, chh = (H + 1) >> 1;
     const int cx0 = x0 / 2 - 1, cy0 = y0 / 2 - 2;
-    static_assert(NR % 4 == 0 && 2 * NR * REST <= 256, "the same work for each wave, a thread for each sample beyond");
+    constexpr int ROWS = (NR + NW - 1) / NW;  // of a wave
+    static_assert(2 * NR * REST <= 64 * NW, "a thread for each sample beyond");
     // all of a thread's loads before its first store
     const int c = tid & 63, r0 = tid >> 6, gx = min(max(cx0 + c, 0), cw - 1);
-    float v[2][NR / 4], beyond = 0.f;
+    float v[2][ROWS], beyond = 0.f;
 #pragma unroll
-    for (int k = 0; k < NR / 4; k++) {
-        const int gy = min(max(cy0 + r0 + 4 * k, 0), chh - 1);
+    for (int k = 0; k < ROWS; k++) {
+        const int gy = min(max(cy0 + r0 + NW * k, 0), chh - 1);
         v[0][k] = sample_u(src[1], stride[1], gx, gy, wide, maxcode);
         v[1][k] = sample_u(src[2], stride[2], gx, gy, wide, maxcode);
     }
@@ -112,9 +113,10 @@ __device__ __forceinline__ void stage_chroma420(float* ch, const uint8_t* const*
     if (tid < NR * REST) beyond = sample_u(src[1], stride[1], bgx, bgy, wide, maxcode);
     else if (tid < 2 * NR * REST) beyond = sample_u(src[2], stride[2], bgx, bgy, wide, maxcode);
 #pragma unroll
-    for (int k = 0; k < NR / 4; k++) {
-        ch[(r0 + 4 * k) * NC + c] = v[0][k];
-        ch[(NR + r0 + 4 * k) * NC + c] = v[1][k];
+    for (int k = 0; k < ROWS; k++) {
+        if (NR % NW && r0 + NW * k >= NR) break;
+        ch[(r0 + NW * k) * NC + c] = v[0][k];
+        ch[(NR + r0 + NW * k) * NC + c] = v[1][k];
     }
     if (tid < 2 * NR * REST) ch[br * NC + bc] = beyond;
 }
