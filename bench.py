@@ -406,17 +406,19 @@ def run_served(a):
     return out, host_pool, alone
 
 
-BUTTER_KERNELS = {"input": "butter_input420_kernel<false>", "opsin": "butter_opsin_kernel", "low": "butter_low_kernel",
-                  "mid": "butter_mid_kernel", "high": "butter_high_kernel", "diff": "butter_diff_kernel",
+BUTTER_KERNELS = {"input": "butter_input420_kernel<false>", "opsin": "butter_strip_kernel<OpsinStage>",
+                  "low": "butter_strip_kernel<LowStage>", "mid": "butter_strip_kernel<MidStage>",
+                  "high": "butter_strip_kernel<HighStage>", "diff": "butter_malta_kernel",
                   "mask": "butter_mask_kernel", "norm": "butter_norm_kernel"}
 BUTTER_BYTES = {"input": "Y + 2 quarter-size chroma bytes read per image, 6 linear FP32 planes written at "
                          "full and quarter size",
-                "opsin": "6 FP32 planes read, 6 written, per pixel of both scales",
-                "low": "6 FP32 planes read, 12 written (low band as values, residual)",
-                "mid": "6 read, 10 written (middle band, high residual)",
-                "high": "4 read, 8 written (high, ultra-high bands)",
-                "diff": "20 read (bands of both images), 4 written (AC, DC sums, 2 mask inputs)",
-                "mask": "4 read, 1 written, plus the half-scale map read at full scale",
+                "opsin": "6 FP32 planes read, 5 written (X and Y of both images, B's difference), per pixel of both "
+                         "scales",
+                "low": "5 FP32 planes read, 6 written (residuals, DC sum)",
+                "mid": "5 read, 7 written (high residuals, 2 Malta differences, AC sum)",
+                "high": "5 read, 7 written (4 Malta differences, AC sum, 2 mask inputs)",
+                "diff": "7 read (6 Malta differences, AC sum), 1 written",
+                "mask": "4 read, plus the half-scale map written and read",
                 "norm": "tile partials"}
 
 
@@ -472,7 +474,8 @@ def run_butter(a):
                                           else "no PMC run of this kernel on this workload"),
                        "kernel": f"{kernel} (both scales, {top} stage)",
                        "algorithmic_bytes_per_launch": int(stage_bytes[top]),
-                       "note": BUTTER_BYTES[top] + "; FP32 stencil sums on the vector ALUs"}
+                       "note": BUTTER_BYTES[top] + ("; blurs on the matrix cores" if top in ("opsin", "low", "mid", "high")
+                                                else "; FP32 stencil sums on the vector ALUs")}
     out["stage_bytes"] = {k: int(v) for k, v in stage_bytes.items()}
     return out, pairs, norms
 

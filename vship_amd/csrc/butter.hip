@@ -24,6 +24,11 @@
 //           map; at full scale also the blend with the half-scale
 //           map and the norm partial sums                        -> map, partials
 //
+// Pairs whose values stay in the range of fp16 parts, all but some float input,
+// take the band stages as strips on the matrix cores instead (butter_strip.hip),
+// which form the differences, L2 terms and mask inputs where the bands are and
+// write no band, and the six Malta terms by butter_malta_kernel.
+//
 // Both images of a pair run in one launch (grid z = pair x image), and a
 // batch of pairs in the same launches; so do both scales, but for the mask:
 // there the half scale runs first, so that the full scale's kernel blends and
@@ -1545,12 +1550,14 @@ uint64_t Engine::stage_bytes(int stage) const {
             b = full * 2 * (1 + 2 * chroma) * bps + full * 6 * 4 + (double)w2_ * h2_ * 6 * 4;
             break;
         }
-        case ST_OPSIN: b = px * (6 + 6) * 4; break;
-        case ST_LOW: b = px * (6 + 12) * 4; break;
-        case ST_MID: b = px * (6 + 10) * 4; break;
-        case ST_HIGH: b = px * (4 + 8) * 4; break;
-        case ST_DIFF: b = px * (20 + 4) * 4; break;
-        case ST_MASK: b = px * (4 + 1) * 4 + (double)w2_ * h2_ * 4; break;
+        // the strip stages and butter_malta_kernel (pairs that the general
+        // kernels score again move more)
+        case ST_OPSIN: b = px * (6 + 5) * 4; break;
+        case ST_LOW: b = px * (5 + 6) * 4; break;
+        case ST_MID: b = px * (5 + 7) * 4; break;
+        case ST_HIGH: b = px * (5 + 7) * 4; break;
+        case ST_DIFF: b = px * (7 + 1) * 4; break;
+        case ST_MASK: b = px * 4 * 4 + (double)w2_ * h2_ * 2 * 4; break;
         default: b = 0.0;
     }
     return (uint64_t)b;

@@ -51,12 +51,12 @@
 // What bounds it is power as much as vector issue: the chip holds about 2 GHz of
 // its 2.4 in it, and less the more matrix products and memory traffic there are.
 // With a wave per strip (each input column split twice: 370 issue slots of the
-// vector unit per 16 x 16 outputs, 24 matrix products) the kernel took 7.35 ms for
-// 240 1080p pairs; with shared windows and 325 slots 6.75 ms. Forms with fewer
-// slots and more products (28, 32) were no faster or slower, and 16 waves of this
-// form per CU read the centre samples from beyond the L2, at a lower clock, for no
-// gain until those came through LDS; twelve waves have the registers to load a
-// window ahead.
+// vector unit per 16 x 16 outputs, 24 matrix products) the kernel took 7.53 ms for
+// 240 1080p pairs; with shared windows and 325 slots 6.66 ms, 87 % of its cycles in
+// vector issue and 26 % with the matrix cores busy. Forms with fewer slots and more
+// products (28, 32) were no faster or slower, and 16 waves of this form per CU read
+// the centre samples from beyond the L2, at a lower clock, for no gain until those
+// came through LDS; twelve waves have the registers to load a window ahead.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 

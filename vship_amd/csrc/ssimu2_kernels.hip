@@ -515,10 +515,10 @@ __device__ __forceinline__ void store_scale1(const PrepLds& L, const PairDev& P,
 // than held across the tile loop, see tid_in_loop), which overlaps one
 // tile's stores with another's arithmetic.
 //
-// What bounds it is its writes (66 MB per 1080p pair, at 4.7 of the 5.6 TB/s a
-// write-only loop reaches), then vector issue. Tiles of 128 x 32 read half as
-// many lines twice as tiles of 64 x 64 (96 1080p pairs 0.98 -> 0.60 million
-// counted reads), a wave's lanes are one row of them, and a tile's samples are
+// What bounds it is its writes (66 MB per 1080p pair, 3.30 ms for 240: 5.0 of the
+// 5.6 TB/s a write-only loop reaches) and vector issue (98 % of its cycles). Tiles
+// of 128 x 32 read fewer lines twice than tiles of 64 x 64 (96 1080p pairs 15.7 ->
+// 9.5 million L2 misses), a wave's lanes are one row of them, and a tile's samples are
 // loaded together, luma before the chroma is staged: one pair after another, as
 // the staging loop had it, the wider tiles were 4 % slower. 240 1080p pairs, the
 // whole batch: 11.02 -> 10.66 ms; 24 pairs of RGB u8, u16, f16, f32: 1,128,
