@@ -47,6 +47,7 @@ enum Stage : int {
 };
 
 struct StripTables;
+struct Tables;
 
 class Engine {
 public:
@@ -95,8 +96,9 @@ private:
     hipStream_t stream_ = nullptr;
     float* arena_ = nullptr;
     int64_t plane0_ = 0, plane1_ = 0;
-    Taps* taps_d_ = nullptr;
-    StripTables* strip_d_ = nullptr;
+    Tables* tables_d_ = nullptr;  // owns the next two
+    const Taps* taps_d_ = nullptr;
+    const StripTables* strip_d_ = nullptr;
     PairDesc* desc_d_ = nullptr;
     PairDesc* desc_h_ = nullptr;
     double* partials_d_ = nullptr;
