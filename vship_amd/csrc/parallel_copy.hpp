@@ -11,6 +11,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -148,8 +149,13 @@ public:
         int64_t dst_stride = 0, src_stride = 0;
     };
 
+    // Fewer helpers, or none, where the system gives no more threads.
     explicit CopyTeam(int helpers) {
-        for (int i = 0; i < helpers; i++) threads_.emplace_back(&CopyTeam::helper, this);
+        threads_.reserve(helpers);
+        try {
+            for (int i = 0; i < helpers; i++) threads_.emplace_back(&CopyTeam::helper, this);
+        } catch (const std::system_error&) {
+        }
     }
     ~CopyTeam() {
         {
