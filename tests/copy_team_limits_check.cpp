@@ -1,9 +1,11 @@
 // CPU checks of CopyTeam (vship_amd/csrc/parallel_copy.hpp) where a machine is
 // short of something; prints "ok" and exits 0 on success.
 //
+//   asleep   while the next chunk is not open, the helpers use no CPU time
 //   threads  a team whose threads the system refuses copies with those it has
 #include <dlfcn.h>
 #include <pthread.h>
+#include <sys/resource.h>
 
 #include <atomic>
 #include <cerrno>
@@ -43,6 +45,30 @@ static bool copied() {
     return same;
 }
 
+static double cpu_seconds() {
+    rusage u;
+    getrusage(RUSAGE_SELF, &u);
+    return (double)(u.ru_utime.tv_sec + u.ru_stime.tv_sec) + 1e-6 * (double)(u.ru_utime.tv_usec + u.ru_stime.tv_usec);
+}
+
+static int asleep() {
+    CopyTeam team(3);
+    const double t0 = cpu_seconds();
+    team.run(
+        pieces(), 2, 2,
+        [](int c, bool wait) {
+            if (c == 0) return true;
+            if (!wait) return false;
+            std::this_thread::sleep_for(std::chrono::milliseconds(500));
+            return true;
+        },
+        [](int) {});
+    const double used = cpu_seconds() - t0;
+    // 2 MiB take about a millisecond; one helper that does not sleep uses the 500
+    std::printf("%.3f s of CPU time\n", used);
+    return copied() && used < 0.1 ? 0 : 1;
+}
+
 static int threads() {
     for (int given = 0; given < 4; given++) {
         g_threads = given;
@@ -59,7 +85,7 @@ static int threads() {
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     for (size_t i = 0; i < src.size(); i++) src[i] = (uint8_t)(i * 2654435761u >> 24);
-    const int rc = what == "threads" ? threads() : 2;
+    const int rc = what == "asleep" ? asleep() : what == "threads" ? threads() : 2;
     if (rc == 0) std::printf("ok\n");
     return rc;
 }

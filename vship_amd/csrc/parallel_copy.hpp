@@ -175,7 +175,6 @@ public:
     // piece. An exception from either ends the copy and is passed on.
     template <class Open, class Done>
     void run(const std::vector<Piece>& pieces, int nchunks, int depth, Open&& open, Done&& done) {
-        Job job(pieces, nchunks);
         std::unique_lock<std::mutex> mine(use_, std::defer_lock);
         if (threads_.empty() || !mine.try_lock()) {
             size_t i = 0;
@@ -186,19 +185,19 @@ public:
             }
             return;
         }
-        post(&job);
+        const auto job = std::make_shared<Job>(pieces, nchunks);
+        post(job);
         int opened = 0;
         try {
             for (int c = 0; c < nchunks; c++) {
-                while (job.left[c].load(std::memory_order_acquire) > 0) {
-                    while (opened < std::min(nchunks, c + depth) && open(opened, opened <= c))
-                        job.opened.store(++opened, std::memory_order_release);
-                    if (!job.take_open(opened)) std::this_thread::yield();
+                while (job->left[c].load(std::memory_order_acquire) > 0) {
+                    while (opened < std::min(nchunks, c + depth) && open(opened, opened <= c)) job->open(++opened);
+                    if (!job->copy_next()) std::this_thread::yield();
                 }
                 done(c);
             }
         } catch (...) {
-            job.abort.store(true);
+            job->drain();
             post(nullptr);
             throw;
         }
@@ -206,36 +205,60 @@ public:
     }
 
 private:
+    // One copy. The helpers share it with the caller and may leave it after the
+    // caller has: no piece is in flight by then.
     struct Job {
-        const std::vector<Piece>& pieces;
+        const std::vector<Piece> pieces;
         std::unique_ptr<std::atomic<int>[]> left;  // pieces of each chunk still to be copied
-        std::atomic<int> next{0}, opened{0};
-        std::atomic<bool> abort{false};
+        std::atomic<int> next{0}, copied{0}, opened{0};
+        std::mutex mu;  // of the sleeping helpers
+        std::condition_variable more;
+        bool over = false;
         Job(const std::vector<Piece>& p, int nchunks) : pieces(p), left(new std::atomic<int>[nchunks]) {
             for (int c = 0; c < nchunks; c++) left[c].store(0, std::memory_order_relaxed);
             for (const Piece& q : p) left[q.chunk].fetch_add(1, std::memory_order_relaxed);
         }
-        void finish(int i) {
+        // copies the next piece, if there is one and its chunk is open
+        bool copy_next() {
+            int i = next.load(std::memory_order_relaxed);
+            do {
+                if (i >= (int)pieces.size() || pieces[i].chunk >= opened.load(std::memory_order_acquire)) return false;
+            } while (!next.compare_exchange_weak(i, i + 1));
             copy(pieces[i]);
             left[pieces[i].chunk].fetch_sub(1, std::memory_order_release);
-        }
-        // the calling thread: one piece, if the next one's chunk is open
-        bool take_open(int open) {
-            int i = next.load(std::memory_order_relaxed);
-            if (i >= (int)pieces.size() || pieces[i].chunk >= open) return false;
-            if (next.compare_exchange_strong(i, i + 1)) finish(i);
+            copied.fetch_add(1, std::memory_order_release);
             return true;
         }
-        // a helper: piece after piece, each when its chunk is open
+        void open(int n) {
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                opened.store(n, std::memory_order_release);
+            }
+            more.notify_all();
+        }
+        // takes the pieces away that nobody has begun, and waits for the others
+        void drain() {
+            const int begun = std::min(next.exchange((int)pieces.size()), (int)pieces.size());
+            while (copied.load(std::memory_order_acquire) < begun) std::this_thread::yield();
+        }
+        void end() {
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                over = true;
+            }
+            more.notify_all();
+        }
+        // A helper: the pieces of open chunks, asleep while there are none. It
+        // takes none before its chunk is open, so that nobody waits for a helper
+        // to wake. (Helpers that waited by yielding kept three CPUs busy while the
+        // caller waited for the link.)
         void help() {
             for (;;) {
-                const int i = next.fetch_add(1);
-                if (i >= (int)pieces.size()) return;
-                while (opened.load(std::memory_order_acquire) <= pieces[i].chunk) {
-                    if (abort.load()) return;
-                    std::this_thread::yield();
-                }
-                finish(i);
+                const int seen = opened.load(std::memory_order_acquire);
+                while (copy_next()) {}
+                std::unique_lock<std::mutex> lk(mu);
+                more.wait(lk, [&] { return over || opened.load(std::memory_order_relaxed) != seen; });
+                if (over) return;
             }
         }
     };
@@ -245,17 +268,15 @@ private:
             std::memcpy(p.dst + (int64_t)r * p.dst_stride, p.src + (int64_t)r * p.src_stride, p.bytes);
     }
 
-    // the job helpers may join; nullptr: none, after the last has left
-    void post(Job* j) {
-        std::unique_lock<std::mutex> lk(mu_);
-        job_ = j;
-        if (j) {
-            gen_++;
-            lk.unlock();
-            go_.notify_all();
-        } else {
-            idle_.wait(lk, [&] { return active_ == 0; });
+    // the job helpers may join, in place of the one before
+    void post(std::shared_ptr<Job> j) {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            job_.swap(j);
+            if (job_) gen_++;
         }
+        if (j) j->end();
+        else go_.notify_all();
     }
 
     void helper() {
@@ -265,22 +286,20 @@ private:
             go_.wait(lk, [&] { return stop_ || (job_ && gen_ != seen); });
             if (stop_) return;
             seen = gen_;
-            Job* j = job_;
-            active_++;
+            std::shared_ptr<Job> j = job_;
             lk.unlock();
             j->help();
+            j.reset();
             lk.lock();
-            if (--active_ == 0) idle_.notify_all();
         }
     }
 
     std::vector<std::thread> threads_;
     std::mutex use_;  // held by the copy that has the helpers
     std::mutex mu_;
-    std::condition_variable go_, idle_;
-    Job* job_ = nullptr;
+    std::condition_variable go_;
+    std::shared_ptr<Job> job_;
     uint64_t gen_ = 0;
-    int active_ = 0;
     bool stop_ = false;
 };
 
