@@ -3,6 +3,7 @@
 //
 //   asleep   while the next chunk is not open, the helpers use no CPU time
 //   threads  a team whose threads the system refuses copies with those it has
+//   taken    taken() says whether a copy has the helpers
 #include <dlfcn.h>
 #include <pthread.h>
 #include <sys/resource.h>
@@ -82,10 +83,32 @@ static int threads() {
     return 0;
 }
 
+static int taken() {
+    CopyTeam team(2), nobody(0);
+    std::atomic<int> bad{0};
+    if (team.taken()) bad++;
+    team.run(
+        pieces(), 2, 2, [](int, bool) { return true; },
+        [&](int) {
+            std::thread([&] {
+                if (!team.taken()) bad++;
+            }).join();
+        });
+    if (team.taken() || !copied()) bad++;
+    nobody.run(
+        pieces(), 2, 2, [](int, bool) { return true; },
+        [&](int) {
+            std::thread([&] {
+                if (nobody.taken()) bad++;  // a copy has nothing that another could want
+            }).join();
+        });
+    return bad ? 1 : 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     for (size_t i = 0; i < src.size(); i++) src[i] = (uint8_t)(i * 2654435761u >> 24);
-    const int rc = what == "asleep" ? asleep() : what == "threads" ? threads() : 2;
+    const int rc = what == "asleep" ? asleep() : what == "threads" ? threads() : what == "taken" ? taken() : 2;
     if (rc == 0) std::printf("ok\n");
     return rc;
 }

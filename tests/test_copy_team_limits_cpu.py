@@ -19,7 +19,7 @@ def check(tmp_path_factory):
 
 
 @pytest.mark.skipif(not shutil.which("g++"), reason="g++ not available")
-@pytest.mark.parametrize("what", ["asleep", "threads"])
+@pytest.mark.parametrize("what", ["asleep", "threads", "taken"])
 def test_copy_team_limits(check, what):
     r = subprocess.run([check, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -90,7 +90,12 @@ std::shared_ptr<CopyTeam> shared_team() {
 // stream itself: a DMA and its hand-over to the kernels behind it cost about
 // 20 us each besides the bytes (measured at 1, 2 and 4 MiB), more than a small
 // picture's whole upload. Bound by PCIe; 64 workgroups keep 256 KiB of 16-byte
-// accesses in flight, several times what the link's latency needs.
+// accesses in flight, several times what the link's latency needs. A copy that
+// finds the helpers taken, as most do where several handles work at once, takes
+// the DMA engines instead: there the link is never idle, and the kernel would
+// only wait for CUs behind the other handles' kernels and hold them up. 1920 x
+// 1080 float Butteraugli with its map, per call: one handle 1,765 us by the
+// kernel and 1,975 by DMA, eight handles on eight threads 1,110 and 965.
 constexpr int kMoveGroups = 64;
 __global__ __launch_bounds__(256) void move_kernel(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src,
                                                    size_t bytes) {
@@ -239,7 +244,9 @@ void HostStager::upload_shared(uint8_t* dst_base, const UploadPlan& plan, hipStr
     if (chunks.empty()) return;
     const int nslots = (int)ring_.size(), n = (int)chunks.size(), first = next_;
     next_ = (first + n) % nslots;
-    team_for(plan.total).run(
+    CopyTeam& team = team_for(plan.total);
+    const bool dma = team.taken();
+    team.run(
         pieces, n, nslots,
         [&](int c, bool wait) {
             // the slot's previous DMA has to have read it before it is refilled
@@ -250,7 +257,11 @@ void HostStager::upload_shared(uint8_t* dst_base, const UploadPlan& plan, hipStr
         },
         [&](int c) {
             const int k = (first + c) % nslots;
-            move_chunk(dst_base + chunks[c].off, ring_[k], chunks[c].bytes, st);
+            void* to = dst_base + chunks[c].off;
+            if (dma)
+                HIP_OR_THROW(hipMemcpyAsync(to, ring_[k], chunks[c].bytes, hipMemcpyHostToDevice, st), E_BadPointer);
+            else
+                move_chunk(to, ring_[k], chunks[c].bytes, st);
             HIP_OR_THROW(hipEventRecord(ev_[k], st), E_BadDeviceCode);
         });
 }
@@ -280,13 +291,15 @@ void HostStager::download_rows(void* dst, int64_t dst_stride, const void* src, i
     const int per = (int)std::min<size_t>(chunk_ / row_bytes, (size_t)rows);
     const int nchunks = (rows + per - 1) / per;
     const int nslots = (int)ring_.size();
-    // chunk c goes through slot (next_ + c) % nslots; up to nslots DMAs ahead
+    CopyTeam& team = team_for(row_bytes * rows);
+    const bool dma = !shared_ || team.taken();
+    // chunk c goes through slot (next_ + c) % nslots; up to nslots ahead
     auto enqueue = [&](int c) {
         const int k = (next_ + c) % nslots;
         const int r0 = c * per, n = std::min(per, rows - r0);
         HIP_OR_THROW(hipEventSynchronize(ev_[k]), E_BadDeviceCode);
         const uint8_t* from = s + (int64_t)r0 * src_stride;
-        if (shared_ && src_stride == (int64_t)row_bytes && reinterpret_cast<uintptr_t>(from) % 16 == 0)
+        if (!dma && src_stride == (int64_t)row_bytes && reinterpret_cast<uintptr_t>(from) % 16 == 0)
             move_chunk(ring_[k], from, row_bytes * n, st);
         else
             HIP_OR_THROW(hipMemcpy2DAsync(ring_[k], row_bytes, from, src_stride, row_bytes, n, hipMemcpyDeviceToHost, st),
@@ -294,7 +307,7 @@ void HostStager::download_rows(void* dst, int64_t dst_stride, const void* src, i
         HIP_OR_THROW(hipEventRecord(ev_[k], st), E_BadDeviceCode);
     };
     for (int c = 0; c < std::min(nchunks, nslots); c++) enqueue(c);
-    // pieces of whole rows, copied out of a chunk once its DMA has arrived
+    // pieces of whole rows, copied out of a chunk once it has arrived
     std::vector<CopyTeam::Piece> pieces;
     const int piece_rows = std::max(1, (int)(kPiece / row_bytes));
     for (int c = 0; c < nchunks; c++)
@@ -320,7 +333,7 @@ void HostStager::download_rows(void* dst, int64_t dst_stride, const void* src, i
     auto copied = [&](int c) {
         if (c + nslots < nchunks) enqueue(c + nslots);
     };
-    team_for(row_bytes * rows).run(pieces, nchunks, nslots, arrived, copied);
+    team.run(pieces, nchunks, nslots, arrived, copied);
     next_ = (next_ + nchunks) % nslots;
     pageable_bytes_ += row_bytes * rows;
 }

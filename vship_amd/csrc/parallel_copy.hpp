@@ -168,6 +168,13 @@ public:
     CopyTeam(const CopyTeam&) = delete;
     CopyTeam& operator=(const CopyTeam&) = delete;
 
+    // Whether a copy has the helpers at this moment.
+    bool taken() {
+        if (threads_.empty()) return false;
+        const std::unique_lock<std::mutex> lk(use_, std::try_to_lock);
+        return !lk.owns_lock();
+    }
+
     // Copies the pieces, which are in order of their chunks 0 .. nchunks - 1,
     // each with at least one piece. On the calling thread, in order:
     // open(c, wait) says whether chunk c may be copied now (wait: blocks until
