@@ -38,6 +38,7 @@
 #include "butter.hpp"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -95,7 +96,7 @@ __device__ __forceinline__ void yuv_rgb(const uint8_t* const* src, const int64_t
 
 template <int FMT>
 __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* __restrict__ pairs, Scale S0,
-                                                                Scale S1, float scale) {
+                                                                Scale S1, float scale, Marks* __restrict__ marks) {
     const int pair = blockIdx.z;
     const int hx = blockIdx.x * 16 + (threadIdx.x & 15), hy = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (hx >= S1.w || hy >= S1.h) return;
@@ -103,6 +104,7 @@ __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* 
     const bool xo = 2 * hx + 1 < w, yo = 2 * hy + 1 < h;
     const int x0 = 2 * hx, y0 = 2 * hy, x1 = xo ? x0 + 1 : x0, y1 = yo ? y0 + 1 : y0;
     const PairDesc& P = pairs[pair];
+    float largest = 0.0f;
     for (int im = 0; im < 2; im++) {
         float v[4][3];  // (x0,y0), (x1,y0), (x0,y1), (x1,y1)
         if constexpr (!fmt_yuv(FMT)) {
@@ -127,6 +129,7 @@ __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* 
         for (int c = 0; c < 3; c++) {
             const float a = linearize(v[0][c]) * scale, b = linearize(v[1][c]) * scale;
             const float cc = linearize(v[2][c]) * scale, d = linearize(v[3][c]) * scale;
+            largest = fmaxf(fmaxf(fmaxf(largest, fabsf(a)), fmaxf(fabsf(b), fabsf(cc))), fabsf(d));
             float* L = plane_of(S0, pair, P_LIN + im * 3 + c);
             L[(int64_t)y0 * S0.pitch + x0] = a;
             if (xo) L[(int64_t)y0 * S0.pitch + x1] = b;
@@ -141,6 +144,10 @@ __global__ __launch_bounds__(kThreads) void butter_input_kernel(const PairDesc* 
             m += d;
             plane_of(S1, pair, P_LIN + im * 3 + c)[(int64_t)hy * S1.pitch + hx] = m * 0.25f;
         }
+    }
+    if constexpr (FMT == IN_RGB_F16 || FMT == IN_RGB_F32) {
+        if (largest > kLinMax) marks[0].general = marks[1 + pair].general = 1;
+        if (largest > FLT_MAX) marks[1 + pair].unscaled = 1;
     }
 }
 
@@ -216,14 +223,15 @@ __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDes
 }
 
 template <int FMT>
-void launch_input(dim3 g, hipStream_t st, const PairDesc* pairs, const Scale& S0, const Scale& S1, float scale) {
-    butter_input_kernel<FMT><<<g, dim3(kThreads), 0, st>>>(pairs, S0, S1, scale);
+void launch_input(dim3 g, hipStream_t st, const PairDesc* pairs, const Scale& S0, const Scale& S1, float scale,
+                  Marks* marks) {
+    butter_input_kernel<FMT><<<g, dim3(kThreads), 0, st>>>(pairs, S0, S1, scale, marks);
 }
 
 template <int... F>
 void launch_input_fmt(int fmt, dim3 g, hipStream_t st, const PairDesc* pairs, const Scale& S0, const Scale& S1,
-                      float scale, std::integer_sequence<int, F...>) {
-    ((fmt == F ? launch_input<F>(g, st, pairs, S0, S1, scale) : void()), ...);
+                      float scale, Marks* marks, std::integer_sequence<int, F...>) {
+    ((fmt == F ? launch_input<F>(g, st, pairs, S0, S1, scale, marks) : void()), ...);
 }
 
 // ---------------------------------------------------------------------------
@@ -490,14 +498,15 @@ __device__ __forceinline__ void blur_tile(BlurLds<R>& L, BlurRegs<R>& S, const f
 }
 
 // sigma 1.2 blur of linear RGB + opsin dynamics (colors.hpp:50-91) -> XYB
-__global__ __launch_bounds__(kThreads) void butter_opsin_kernel(Scales SS, int nz, const Taps* __restrict__ taps,
+__global__ __launch_bounds__(kThreads) void butter_opsin_kernel(Scales SS, int nz, const int32_t* __restrict__ which,
+                                                                const Taps* __restrict__ taps,
                                                                 float intensity) {
     constexpr int R = kRad[SG_OPSIN];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_OPSIN;
     Scale S;
     const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
-    const int pair = ti.z >> 1, im = ti.z & 1;
+    const int pair = which[ti.z >> 1], im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     edge_factors<R, kTW, kTH>(L.colf, L.rowf, T, S.w, S.h, ox0, oy0);
     float bl[3][kRun], ctr[3][kRun];
@@ -529,13 +538,14 @@ __global__ __launch_bounds__(kThreads) void butter_opsin_kernel(Scales SS, int n
 
 // sigma 7.156 blur: low band (stored as values, XybLowFreqToVals) and the
 // residual XYB - low (separatefrequencies.hpp:142-170)
-__global__ __launch_bounds__(kThreads) void butter_low_kernel(Scales SS, int nz, const Taps* __restrict__ taps) {
+__global__ __launch_bounds__(kThreads) void butter_low_kernel(Scales SS, int nz, const int32_t* __restrict__ which,
+                                                              const Taps* __restrict__ taps) {
     constexpr int R = kRad[SG_LOW];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_LOW;
     Scale S;
     const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
-    const int pair = ti.z >> 1, im = ti.z & 1;
+    const int pair = which[ti.z >> 1], im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     const RunPos p = run_pos();
     const int gx = ox0 + p.tx, gy = oy0 + p.ty;
@@ -569,13 +579,14 @@ __global__ __launch_bounds__(kThreads) void butter_low_kernel(Scales SS, int nz,
 // sigma 3.225 blur of the residual: middle band after its range operation,
 // high residual = residual - middle band, X's residual suppressed by Y's
 // (separatefrequencies.hpp:160-189)
-__global__ __launch_bounds__(kThreads) void butter_mid_kernel(Scales SS, int nz, const Taps* __restrict__ taps) {
+__global__ __launch_bounds__(kThreads) void butter_mid_kernel(Scales SS, int nz, const int32_t* __restrict__ which,
+                                                              const Taps* __restrict__ taps) {
     constexpr int R = kRad[SG_MID];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_MID;
     Scale S;
     const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
-    const int pair = ti.z >> 1, im = ti.z & 1;
+    const int pair = which[ti.z >> 1], im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     const RunPos p = run_pos();
     const int gx = ox0 + p.tx, gy = oy0 + p.ty;
@@ -613,13 +624,14 @@ __global__ __launch_bounds__(kThreads) void butter_mid_kernel(Scales SS, int nz,
 
 // sigma 1.564 blur of the high residual: high and ultra-high bands
 // (separatefrequencies.hpp:117-140, 190-200)
-__global__ __launch_bounds__(kThreads) void butter_high_kernel(Scales SS, int nz, const Taps* __restrict__ taps) {
+__global__ __launch_bounds__(kThreads) void butter_high_kernel(Scales SS, int nz, const int32_t* __restrict__ which,
+                                                               const Taps* __restrict__ taps) {
     constexpr int R = kRad[SG_HIGH];
     __shared__ BlurLds<R> L;
     const Taps* T = taps + SG_HIGH;
     Scale S;
     const TileIdx ti = tile_of_scales<kTW, kTH>(SS, nz, S);
-    const int pair = ti.z >> 1, im = ti.z & 1;
+    const int pair = which[ti.z >> 1], im = ti.z & 1;
     const int ox0 = ti.x * kTW, oy0 = ti.y * kTH;
     const RunPos p = run_pos();
     const int gx = ox0 + p.tx, gy = oy0 + p.ty;
@@ -742,11 +754,12 @@ __device__ __forceinline__ void malta_block(const float* __restrict__ win_origin
     }
 }
 
-__global__ __launch_bounds__(kThreads) void butter_diff_kernel(Scales SS, int nz, DiffParams D) {
+__global__ __launch_bounds__(kThreads) void butter_diff_kernel(Scales SS, int nz, const int32_t* __restrict__ which,
+                                                               DiffParams D) {
     __shared__ float dt[kDSH * kDSW];
     Scale S;
     const TileIdx ti = tile_of_scales<kDW, kDH>(SS, nz, S);
-    const int pair = ti.z;
+    const int pair = which[ti.z];
     const int ox0 = ti.x * kDW, oy0 = ti.y * kDH;
     const int tx = threadIdx.x & (kDW - 1), ty = threadIdx.x / kDW;
     const int w = S.w, h = S.h;
@@ -982,7 +995,9 @@ __device__ __forceinline__ void malta_sums(const float* __restrict__ win_origin,
 // sums, in two LDS buffers (one barrier per term). Three waves per SIMD hold the
 // window and the shared segments (142 registers): held to four waves the
 // kernel spills and took 0.71 ms instead of 0.66, to five 0.80.
-__global__ __launch_bounds__(kThreads, 3) void butter_malta_kernel(Scales SS, int nz) {
+__global__ __launch_bounds__(kThreads, 3) void butter_malta_kernel(Scales SS, int nz,
+                                                                   const Marks* __restrict__ marks) {
+    const int any = marks->general;
     constexpr int kVec = kDSW / 4, kLoads = (kVec * kDSH + kThreads - 1) / kThreads;
     static_assert(kDSW % 4 == 0 && kDHalo % 4 == 0, "16-byte loads");
     __shared__ float4 dt[2][kDSH * kVec];
@@ -1013,6 +1028,7 @@ __global__ __launch_bounds__(kThreads, 3) void butter_malta_kernel(Scales SS, in
         for (int k = 0; k < kLoads; k++) v[k] = *reinterpret_cast<const float4*>(&at(const_cast<float*>(a), off[k]));
     };
     load(0);
+    if (any && marks[1 + pair].general) return;
     float ac[kDRows];
 #pragma unroll
     for (int j = 0; j < kDRows; j++) ac[j] = 0.0f;
@@ -1089,6 +1105,8 @@ struct NormArgs {
     double* partials;  // [pair][tile][3]
     int tiles;
     const PairDesc* pairs;
+    const Marks* marks;    // for the strips' pairs: to leave the general kernels' out
+    const int32_t* which;  // for those (FAR): the pairs
     const float* half_map_base;  // half-scale P_MAP of pair 0
     int64_t half_pair;           // floats between pairs in the half scale
     int half_pitch;              // floats between rows in the half scale
@@ -1105,14 +1123,15 @@ __device__ __forceinline__ double wave_max(double v) {
     return v;
 }
 
-template <bool FULL>
+template <bool FULL, bool FAR>
 __global__ __launch_bounds__(kThreads) void butter_mask_kernel(Scale S, const Taps* __restrict__ taps, NormArgs N) {
+    const int any = FAR ? 0 : N.marks->general;
     using M = MaskLds;
     constexpr int R = M::R;
     __shared__ MaskLds L;
     const Taps* T = taps + SG_MASK;
     const TileIdx ti = tile_of_block();
-    const int pair = ti.z;
+    const int pair = FAR ? N.which[ti.z] : ti.z;
     const int ox0 = ti.x * kMT, oy0 = ti.y * kMT;
     const int w = S.w, h = S.h;
     edge_factors<R, kMB, kMB>(L.colf, L.rowf, T, w, h, ox0 - kMF, oy0 - kMF);
@@ -1132,6 +1151,7 @@ __global__ __launch_bounds__(kThreads) void butter_mask_kernel(Scale S, const Ta
         half_in[j] = (FULL && ok) ? N.half_map_base[(int64_t)pair * N.half_pair + (int64_t)(gy / 2) * N.half_pitch + gx / 2]
                                   : 0.0f;
     }
+    if (any && N.marks[1 + pair].general) return;
     // blurred reference mask on the 40 x 40 region
     stage_padded<M::SW, M::SWP, M::SW>(L.in, plane_u(S, pair, P_M0), w, h, S.pitch, ox0 - kMF - R, oy0 - kMF - R);
     __syncthreads();
@@ -1228,14 +1248,14 @@ __global__ __launch_bounds__(kThreads) void butter_mask_kernel(Scale S, const Ta
     }
 }
 
-// norms of each pair from its tile partials (diffnorms.hpp:85-127), and whether
-// it has to be scored again by the general kernels
+// norms of each pair from its tile partials (diffnorms.hpp:85-127), and its marks
 __global__ __launch_bounds__(kThreads) void butter_norm_kernel(const double* __restrict__ partials, int tiles,
                                                                int qnorm, int64_t npix,
-                                                               const PairDesc* __restrict__ pairs,
+                                                               const Marks* __restrict__ marks,
+                                                               const int32_t* __restrict__ which,
                                                                double* __restrict__ norms) {
     __shared__ double red[3][kThreads / 64];
-    const int pair = blockIdx.x;
+    const int pair = which ? which[blockIdx.x] : blockIdx.x;
     const double* p = partials + (int64_t)pair * tiles * 3;
     double a = 0.0, b = 0.0, m = 0.0;
     for (int i = threadIdx.x; i < tiles; i += kThreads) {
@@ -1263,7 +1283,7 @@ __global__ __launch_bounds__(kThreads) void butter_norm_kernel(const double* __r
         norms[4 * pair + 0] = pow(sa / (double)npix, 1.0 / (double)qnorm);
         norms[4 * pair + 1] = pow(sb / (double)npix, 1.0 / 3.0);
         norms[4 * pair + 2] = sm;
-        norms[4 * pair + 3] = (double)pairs[pair].general;
+        norms[4 * pair + 3] = (double)(marks[1 + pair].general + 2 * marks[1 + pair].unscaled);
     }
 }
 
@@ -1300,6 +1320,11 @@ DiffParams diff_params() {
 }
 
 }  // namespace
+
+// The block of a call's n pairs: Marks [1 + n], indices of the general kernels'
+// pairs [n], descriptors [n].
+static size_t which_offset(int n) { return sizeof(Marks) * (1 + (size_t)n); }
+static size_t desc_offset(int n) { return (which_offset(n) + sizeof(int32_t) * (size_t)n + 63) / 64 * 64; }
 
 uint64_t Engine::pair_bytes(int width, int height) {
     const int w2 = (width - 1) / 2 + 1, h2 = (height - 1) / 2 + 1;
@@ -1354,8 +1379,9 @@ Engine::Engine(int width, int height, int capacity, int qnorm, float intensity, 
         HIP_OR_THROW(hipMalloc(&partials_d_, sizeof(double) * 3 * mask_tiles_ * cap_), E_OutOfVRAM);
         HIP_OR_THROW(hipMalloc(&norms_d_, sizeof(double) * 4 * cap_), E_OutOfVRAM);
         HIP_OR_THROW(hipHostMalloc(&norms_h_, sizeof(double) * 4 * cap_), E_OutOfRAM);
-        HIP_OR_THROW(hipMalloc(&desc_d_, sizeof(PairDesc) * cap_), E_OutOfVRAM);
-        HIP_OR_THROW(hipHostMalloc(&desc_h_, sizeof(PairDesc) * cap_), E_OutOfRAM);
+        const size_t block = desc_offset(cap_) + sizeof(PairDesc) * cap_;
+        HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&block_d_), block), E_OutOfVRAM);
+        HIP_OR_THROW(hipHostMalloc(reinterpret_cast<void**>(&block_h_), block), E_OutOfRAM);
         HIP_OR_THROW(hipMalloc(&tables_d_, sizeof(Tables)), E_OutOfVRAM);
         HIP_OR_THROW(hipMemcpy(tables_d_, &tables(), sizeof(Tables), hipMemcpyHostToDevice), E_BadDeviceArgument);
         strip_d_ = &tables_d_->strip;
@@ -1377,8 +1403,8 @@ void Engine::release() {
     if (partials_d_) (void)hipFree(partials_d_), partials_d_ = nullptr;
     if (norms_d_) (void)hipFree(norms_d_), norms_d_ = nullptr;
     if (norms_h_) (void)hipHostFree(norms_h_), norms_h_ = nullptr;
-    if (desc_d_) (void)hipFree(desc_d_), desc_d_ = nullptr;
-    if (desc_h_) (void)hipHostFree(desc_h_), desc_h_ = nullptr;
+    if (block_d_) (void)hipFree(block_d_), block_d_ = nullptr;
+    if (block_h_) (void)hipHostFree(block_h_), block_h_ = nullptr;
     if (tables_d_) (void)hipFree(tables_d_), tables_d_ = nullptr;
     if (stream_) (void)hipStreamDestroy(stream_), stream_ = nullptr;
 }
@@ -1418,64 +1444,74 @@ void Engine::run(int fmt, const PairDesc* pairs, int n, double* norms) {
     for (int i = 0; i < n && staged420_; i++) staged420_ = pairs[i].cloc == CLOC_LEFT;
     last_fmt_ = fmt;
     last_n_ = n;
-    score(fmt, pairs, n, false);
-    // a pair with values beyond the range of the matrix-core stages is scored
-    // by the general kernels
-    std::vector<PairDesc> again;
-    std::vector<int> which;
-    for (int i = 0; i < n; i++) {
-        if (norms) std::memcpy(norms + 3 * i, norms_h_ + 4 * i, sizeof(double) * 3);
-        if (norms_h_[4 * i + 3] != 0.0) {
-            again.push_back(pairs[i]);
-            which.push_back(i);
-        }
-    }
-    if (again.empty()) return;
-    score(fmt, again.data(), (int)again.size(), true);
-    for (size_t k = 0; norms && k < which.size(); k++)
-        std::memcpy(norms + 3 * which[k], norms_h_ + 4 * k, sizeof(double) * 3);
-}
-
-void Engine::score(int fmt, const PairDesc* pairs, int n, bool general) {
-    // a batch that ended in an error may still read the pinned descriptors
+    // a batch that ended in an error may still read the pinned block
     if (in_flight_) HIP_OR_THROW(hipStreamSynchronize(stream_), E_BadDeviceArgument);
     in_flight_ = true;
-    std::memcpy(desc_h_, pairs, sizeof(PairDesc) * n);
-    for (int i = 0; i < n; i++) desc_h_[i].general = 0;
-    HIP_OR_THROW(hipMemcpyAsync(desc_d_, desc_h_, sizeof(PairDesc) * n, hipMemcpyHostToDevice, stream_),
-                 E_BadDeviceArgument);
-    launch(fmt, n, general);
+    const size_t at = desc_offset(n), bytes = at + sizeof(PairDesc) * n;
+    std::memset(block_h_, 0, at);
+    std::memcpy(block_h_ + at, pairs, sizeof(PairDesc) * n);
+    HIP_OR_THROW(hipMemcpyAsync(block_d_, block_h_, bytes, hipMemcpyHostToDevice, stream_), E_BadDeviceArgument);
+    launch(fmt, n, 0, false);
+    fetch_norms(n);
+    // Pairs with values beyond the matrix-core stages are the general kernels',
+    // which read the linear planes that are there.
+    int32_t* const which = reinterpret_cast<int32_t*>(block_h_ + which_offset(n));
+    int far = 0;
+    bool unscaled = false;
+    for (int i = 0; i < n; i++) {
+        if (norms_h_[4 * i + 3] != 0.0) which[far++] = i;
+        unscaled = unscaled || norms_h_[4 * i + 3] >= 2.0;
+    }
+    if (far) {
+        HIP_OR_THROW(hipMemcpyAsync(block_d_ + which_offset(n), which, sizeof(int32_t) * far, hipMemcpyHostToDevice,
+                                    stream_),
+                     E_BadDeviceArgument);
+        launch(fmt, n, far, unscaled);
+        fetch_norms(n);
+    }
+    in_flight_ = false;
+    for (int i = 0; norms && i < n; i++) std::memcpy(norms + 3 * i, norms_h_ + 4 * i, sizeof(double) * 3);
+}
+
+void Engine::fetch_norms(int n) {
     HIP_OR_THROW(hipMemcpyAsync(norms_h_, norms_d_, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, stream_),
                  E_BadDeviceArgument);
     HIP_OR_THROW(hipStreamSynchronize(stream_), E_BadDeviceArgument);
-    in_flight_ = false;
 }
 
-void Engine::launch(int fmt, int n, bool general) {
+void Engine::launch(int fmt, int pairs, int far, bool unscaled) {
+    const bool general = far > 0;
+    const int n = general ? far : pairs;
     const Scale S0{arena_, w_, h_, row_pitch(w_), plane0_, (int64_t)P_COUNT * plane0_};
     const Scale S1{arena_ + (int64_t)cap_ * P_COUNT * plane0_, w2_, h2_, row_pitch(w2_), plane1_,
                    (int64_t)P_COUNT * plane1_};
+    Marks* const marks = reinterpret_cast<Marks*>(block_d_);
+    const int32_t* const which = general ? reinterpret_cast<const int32_t*>(block_d_ + which_offset(pairs)) : nullptr;
+    const PairDesc* const desc = reinterpret_cast<const PairDesc*>(block_d_ + desc_offset(pairs));
+    // the scale of the linear planes: a power of two, which the general kernels'
+    // blur carries exactly and their intensity takes back
+    const float lin = unscaled ? 1.0f : kLinScale;
     StripArgs A;
-    A.pairs = desc_d_;
-    A.intensity = intensity_ / kLinScale;
+    A.marks = marks;
+    A.intensity = intensity_ / lin;
     A.diff = diff_params();
-    const float lin = general ? 1.0f : kLinScale;
     const int th = strip_height(w_, h_, w2_, h2_, n);
     const bool prof = profile_;
     auto mark = [&](int st) {
         if (prof) (void)hipEventRecord(ev_[st], stream_);
     };
-    const dim3 gi(cdiv(w2_, 16), cdiv(h2_, 16), n);
-    auto input = [&] {
+    const dim3 gi(cdiv(w2_, 16), cdiv(h2_, 16), pairs);
+    auto convert = [&] {
         if (staged420_) {
-            const dim3 g4(cdiv(w_, kInputW), cdiv(h_, kInputH), n);
+            const dim3 g4(cdiv(w_, kInputW), cdiv(h_, kInputH), pairs);
             if (fmt == IN_YUV420_U16)
-                butter_input420_kernel<true><<<g4, dim3(kThreads), 0, stream_>>>(desc_d_, S0, S1, lin);
+                butter_input420_kernel<true><<<g4, dim3(kThreads), 0, stream_>>>(desc, S0, S1, lin);
             else
-                butter_input420_kernel<false><<<g4, dim3(kThreads), 0, stream_>>>(desc_d_, S0, S1, lin);
+                butter_input420_kernel<false><<<g4, dim3(kThreads), 0, stream_>>>(desc, S0, S1, lin);
             return;
         }
-        launch_input_fmt(fmt, gi, stream_, desc_d_, S0, S1, lin, std::make_integer_sequence<int, IN_NUM_FORMATS>{});
+        launch_input_fmt(fmt, gi, stream_, desc, S0, S1, lin, marks,
+                         std::make_integer_sequence<int, IN_NUM_FORMATS>{});
     };
     const Scales SS{{S0, S1}};
     // workgroups of a two-scale launch with tiles of tw x th and nz plane sets
@@ -1487,20 +1523,23 @@ void Engine::launch(int fmt, int n, bool general) {
         N.qnorm = q_;
         N.partials = partials_d_;
         N.tiles = mask_tiles_;
-        N.pairs = desc_d_;
+        N.pairs = desc;
+        N.marks = marks;
+        N.which = which;
         N.half_map_base = S1.base + (int64_t)P_MAP * S1.plane;
         N.half_pair = S1.pair;
         N.half_pitch = S1.pitch;
         const dim3 gm(cdiv(S.w, kMT), cdiv(S.h, kMT), n);
-        if (full)
-            butter_mask_kernel<true><<<gm, dim3(kThreads), 0, stream_>>>(S, taps_d_, N);
-        else
-            butter_mask_kernel<false><<<gm, dim3(kThreads), 0, stream_>>>(S, taps_d_, N);
+        auto* k = full ? (general ? butter_mask_kernel<true, true> : butter_mask_kernel<true, false>)
+                       : (general ? butter_mask_kernel<false, true> : butter_mask_kernel<false, false>);
+        k<<<gm, dim3(kThreads), 0, stream_>>>(S, taps_d_, N);
     };
     auto stage = [&](int st) {
         const dim3 blk(kThreads);
         switch (st) {
-            case ST_INPUT: input(); break;
+            case ST_INPUT:
+                if (!general || unscaled) convert();
+                break;
             case ST_OPSIN:
             case ST_LOW:
             case ST_MID:
@@ -1510,17 +1549,17 @@ void Engine::launch(int fmt, int n, bool general) {
                     break;
                 }
                 const dim3 g = grid2(kTW, kTH, 2 * n);
-                if (st == ST_OPSIN) butter_opsin_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_, intensity_);
-                if (st == ST_LOW) butter_low_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_);
-                if (st == ST_MID) butter_mid_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_);
-                if (st == ST_HIGH) butter_high_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, taps_d_);
+                if (st == ST_OPSIN) butter_opsin_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, which, taps_d_, A.intensity);
+                if (st == ST_LOW) butter_low_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, which, taps_d_);
+                if (st == ST_MID) butter_mid_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, which, taps_d_);
+                if (st == ST_HIGH) butter_high_kernel<<<g, blk, 0, stream_>>>(SS, 2 * n, which, taps_d_);
                 break;
             }
             case ST_DIFF:
                 if (general)
-                    butter_diff_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n, A.diff);
+                    butter_diff_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n, which, A.diff);
                 else
-                    butter_malta_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n);
+                    butter_malta_kernel<<<grid2(kDW, kDH, n), blk, 0, stream_>>>(SS, n, marks);
                 break;
             case ST_MASK:
                 mask(S1, false);  // the full scale blends its map with this one's
@@ -1528,7 +1567,7 @@ void Engine::launch(int fmt, int n, bool general) {
                 break;
             default:
                 butter_norm_kernel<<<dim3(n), blk, 0, stream_>>>(partials_d_, mask_tiles_, q_, (int64_t)w_ * h_,
-                                                                 desc_d_, norms_d_);
+                                                                 marks, which, norms_d_);
         }
     };
     for (int st = 0; st < ST_COUNT; st++) {

@@ -30,7 +30,19 @@ struct PairDesc {
     int32_t bits;
     int32_t cloc;
     float kr, kb;
-    int32_t general;  // set by the kernels: a value beyond the range of the matrix-core stages
+};
+
+// What the kernels find out about a pair. One whose values the matrix-core
+// stages cannot hold is left out by every later launch of theirs, and the
+// general kernels score it. The marks of the pairs follow one that says whether
+// any is general: a workgroup reads that one while it works out its tile, and
+// its pair's only then (read by every workgroup, the pairs' marks took the Malta
+// and mask kernels 1 to 3 % longer). Sixteen 1080p pairs with a far sample each
+// take 5.7 ms (the general kernels alone 5.0, 3.6 ms without such samples); with
+// every stage of the strips first they took 9.1.
+struct Marks {
+    int32_t general;   // a value beyond the matrix-core stages
+    int32_t unscaled;  // infinite linear RGB times kLinScale: the general kernels need it as it is
 };
 
 // Kernel groups, for per-kernel timing.
@@ -79,9 +91,11 @@ public:
     static uint64_t pair_bytes(int width, int height);
 
 private:
-    // Uploads the descriptors, runs every stage and waits for the norms.
-    void score(int fmt, const PairDesc* pairs, int n, bool general);
-    void launch(int fmt, int n, bool general);
+    // Every stage on the device: of all pairs on the matrix cores (far 0), or of
+    // the far ones by the general kernels (unscaled: with the planes of linear
+    // RGB made again, without their factor).
+    void launch(int fmt, int pairs, int far, bool unscaled);
+    void fetch_norms(int n);  // waits for them
     void release();
 
     int w_, h_, w2_, h2_, cap_, q_;
@@ -99,8 +113,8 @@ private:
     Tables* tables_d_ = nullptr;  // owns the next two
     const Taps* taps_d_ = nullptr;
     const StripTables* strip_d_ = nullptr;
-    PairDesc* desc_d_ = nullptr;
-    PairDesc* desc_h_ = nullptr;
+    uint8_t* block_d_ = nullptr;  // marks and descriptors of a call's pairs
+    uint8_t* block_h_ = nullptr;
     double* partials_d_ = nullptr;
     double* norms_d_ = nullptr;
     double* norms_h_ = nullptr;

@@ -30,11 +30,12 @@
 // of 256 x 256 pairs were 0.65e-6 from their 64-bit values on average, now
 // 0.40e-6 (vector kernels 0.69e-6), for 0.5 % of the time of a batch. fp16 ends at 65,504, and inputs are not bounded by nature (float RGB;
 // chroma far outside the gamut next to its opposite, at a high intensity):
-// the opsin stage checks every sample and every result against kLinMax and
-// kXybMax, below which no later value leaves the range (XYB minus its low
-// band is below 2 kXybMax, minus its middle band below 4 kXybMax = 32,768). A
-// pair that fails, NaN included, is marked, and the engine scores it again
-// with the general kernels.
+// the input kernels check float samples against kLinMax (those of the other
+// formats are below 10, of 32), and the opsin stage its results against kXybMax,
+// below which no later value leaves the range (XYB minus its low band is below 2
+// kXybMax, minus its middle band below 4 kXybMax = 32,768). A pair that fails,
+// NaN included, is marked; the stages from there on leave it out, and the
+// general kernels score it.
 #include <cmath>
 #include <cstring>
 
@@ -56,7 +57,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kTapScale = 16384.0f;
-constexpr float kLinMax = 32768.0f;  // of linear RGB times kLinScale
 constexpr float kXybMax = 8192.0f;
 
 // ---------------------------------------------------------------------------
@@ -250,16 +250,14 @@ struct OpsinStage {
                 y[k] = o0 + o1;
                 z[im][k] = o2;
                 // o0, o1 and o2 are positive, so the sums bound X, Y and B
-                const bool in = fabsf(ctr[0][k]) <= kLinMax && fabsf(ctr[1][k]) <= kLinMax &&
-                                fabsf(ctr[2][k]) <= kLinMax && y[k] <= kXybMax && o2 <= kXybMax;
-                ok = ok && (in || (k == 1 && !X.two));
+                ok = ok && ((y[k] <= kXybMax && o2 <= kXybMax) || (k == 1 && !X.two));
             }
             put2<NT>(plane_u(S, pair, Q_XY + 2 * im), X.g, x);
             put2<NT>(plane_u(S, pair, Q_XY + 2 * im + 1), X.g, y);
         }
         const float d[2] = {z[0][0] - z[1][0], z[0][1] - z[1][1]};
         put2<NT>(plane_u(S, pair, Q_DB), X.g, d);
-        if (!ok) A.pairs[pair].general = 1;
+        if (!ok) A.marks[0].general = A.marks[1 + pair].general = 1;
     }
 };
 
@@ -450,6 +448,7 @@ template <class K, bool NT>
 __global__ __launch_bounds__(kThreads, K::kWaves) void butter_strip_kernel(Scales SS, int npairs, int th,
                                                                            const StripTables* __restrict__ tab,
                                                                            StripArgs A) {
+    const int any = A.marks->general;
     constexpr int R = K::R, P = K::kPlanes;
     // planes beyond the fourth: a 16-column half for each wave (two planes), or
     // for the even or the odd waves (one), in turn by workgroup
@@ -469,6 +468,7 @@ __global__ __launch_bounds__(kThreads, K::kWaves) void butter_strip_kernel(Scale
                             : tile_of(blockIdx.x, nx0, ny0, npairs);
     const int pair = ti.z, x0 = ti.x * kStripW, y0 = ti.y * th;
     const int w = S.w, h = S.h, pitch = S.pitch;
+    if (any && A.marks[1 + pair].general) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int g = lane >> 4, j = lane & 15;
     auto& in = lds[wave];

@@ -10,6 +10,7 @@ namespace bt {
 
 constexpr int kStripW = 32;           // columns of a strip
 constexpr float kLinScale = 1024.0f;  // of linear RGB in the work planes these stages read
+constexpr float kLinMax = 32768.0f;   // the largest magnitude there, as stored
 
 // Work planes of the matrix-core stages, in the same arena as the general
 // kernels' (the AC and DC sums, the mask inputs and the map are shared).
@@ -33,7 +34,7 @@ struct StripTables {
 void fill_strip_tables(StripTables& T);
 
 struct StripArgs {
-    PairDesc* pairs;
+    Marks* marks;
     float intensity;  // of linear RGB as stored (times kLinScale)
     DiffParams diff;
 };
