@@ -125,8 +125,8 @@ __device__ __forceinline__ TileIdx tile_of_scales(const Scales& SS, int nz, Scal
 
 // 1 / (sum of the taps inside [0, n)) at position p in [0, n) for a window of
 // radius R (gaussianblur.hpp:63-65, 83-84).
-template <int R>
-__device__ __forceinline__ float inv_total(const Taps* __restrict__ T, int p, int n) {
+template <int R, class Sums>
+__device__ __forceinline__ float inv_total(const Sums* __restrict__ T, int p, int n) {
     const int lo = max(0, R - p), hi = min(2 * R, n - 1 - p + R);
     return 1.0f / (T->cum[hi + 1] - T->cum[lo]);
 }

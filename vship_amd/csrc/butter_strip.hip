@@ -160,9 +160,11 @@ __device__ __forceinline__ f32x4 mma(const Op& a, const Op& b, f32x4 c) {
     return mfma32(a.h, b.h, c);
 }
 // An operand of which only the first four of each lane's eight values have
-// taps (the taps' other four are 0). One instruction shape throughout: a
-// 16x16x16 product that accumulates onto a 16x16x32 one right before it read
-// the first two of its four accumulators too early.
+// taps (the taps' other four are 0). One instruction shape throughout: with a
+// 16x16x16 product accumulating onto a 16x16x32 one right before it, the results
+// were wrong in two of the four accumulators under some schedules. The compiler
+// (clang 22 of ROCm 7.2) puts no wait between the two, as between two products of
+// one shape; whether the hardware asks for one there is not known here.
 __device__ __forceinline__ Op half_op(const Half& a) {
     return {u32x4{a.h[0], a.h[1], a.h[0], a.h[1]}, u32x4{a.l[0], a.l[1], a.l[0], a.l[1]}};
 }
@@ -228,7 +230,8 @@ __device__ __forceinline__ void load_centres(Centres<P>& C, const Scale& S, int 
 // both images, and the difference of the two Bs, all that the later stages
 // need of it (they are linear in B)
 struct OpsinStage {
-    static constexpr int R = 8, kSig = SG_OPSIN, kPlanes = 6, kSrc = Q_LIN, kCentres = 6, kWaves = 4;
+    static constexpr int R = 8, kPlanes = 6, kSrc = Q_LIN, kCentres = 6, kWaves = 4;
+    static constexpr StripTables::Blur StripTables::*kBlur = &StripTables::opsin;
     template <bool NT>
     static __device__ __forceinline__ void points(const Exchange<6>& E, const Px& X, const Centres<6>& C,
                                                   const Scale& S, int pair, const StripArgs& A) {
@@ -264,7 +267,8 @@ struct OpsinStage {
 // sigma 7.156 blur: residual XYB - low band, and the L2 terms of the low
 // bands as values (separatefrequencies.hpp:142-170, 3-13; simplerdiff.hpp:38-58)
 struct LowStage {
-    static constexpr int R = 21, kSig = SG_LOW, kPlanes = 5, kSrc = Q_XY, kCentres = 5, kWaves = 3;
+    static constexpr int R = 21, kPlanes = 5, kSrc = Q_XY, kCentres = 5, kWaves = 3;
+    static constexpr StripTables::Blur StripTables::*kBlur = &StripTables::low;
     template <bool NT>
     static __device__ __forceinline__ void points(const Exchange<5>& E, const Px& X, const Centres<5>& C,
                                                   const Scale& S, int pair, const StripArgs&) {
@@ -291,7 +295,8 @@ struct LowStage {
 // operations, as Malta differences and L2 terms; high residual, X's
 // suppressed by Y's (separatefrequencies.hpp:160-189)
 struct MidStage {
-    static constexpr int R = 9, kSig = SG_MID, kPlanes = 5, kSrc = Q_T, kCentres = 4, kWaves = 3;
+    static constexpr int R = 9, kPlanes = 5, kSrc = Q_T, kCentres = 4, kWaves = 3;
+    static constexpr StripTables::Blur StripTables::*kBlur = &StripTables::mid;
     template <bool NT>
     static __device__ __forceinline__ void points(const Exchange<5>& E, const Px& X, const Centres<4>& C,
                                                   const Scale& S, int pair, const StripArgs& A) {
@@ -332,7 +337,8 @@ struct MidStage {
 // differences, L2 terms and mask inputs (separatefrequencies.hpp:117-140,
 // 190-200; simplerdiff.hpp:60-101; maskPsycho.hpp:24-40)
 struct HighStage {
-    static constexpr int R = 8, kSig = SG_HIGH, kPlanes = 4, kSrc = Q_HFR, kCentres = 4, kWaves = 4;
+    static constexpr int R = 8, kPlanes = 4, kSrc = Q_HFR, kCentres = 4, kWaves = 4;
+    static constexpr StripTables::Blur StripTables::*kBlur = &StripTables::high;
     template <bool NT>
     static __device__ __forceinline__ void points(const Exchange<4>& E, const Px& X, const Centres<4>& C,
                                                   const Scale& S, int pair, const StripArgs& A) {
@@ -487,13 +493,13 @@ __global__ __launch_bounds__(kThreads, K::kWaves) void butter_strip_kernel(Scale
     }
 
     Op rop[N::kRow], cop[N::kCol];
-    const u32x4* ops = reinterpret_cast<const u32x4*>(tab->op[K::kSig]);
+    const StripTables::Blur* T = &(tab->*K::kBlur);
+    const u32x4* ops = reinterpret_cast<const u32x4*>(T->op);
 #pragma unroll
     for (int i = 0; i < N::kRow; i++) rop[i] = {ops[2 * i * 64 + lane], ops[(2 * i + 1) * 64 + lane]};
 #pragma unroll
     for (int i = 0; i < N::kCol; i++)
         cop[i] = {ops[2 * (N::kRow + i) * 64 + lane], ops[(2 * (N::kRow + i) + 1) * 64 + lane]};
-    const Taps* T = &tab->taps[K::kSig];
     const float full = 1.0f / T->cum[2 * R + 1] * (1.0f / kTapScale);
     float kcol[kUnits];
 #pragma unroll
@@ -618,7 +624,7 @@ void launch(const Scales& SS, int n, int th, const StripTables* tab, const Strip
 }
 
 template <int R>
-void fill(StripTables& T, int sig) {
+void fill(StripTables::Blur& T, int sig) {
     double g[2 * R + 1], tot = 0.0, run = 0.0;
     uint16_t hi[2 * R + 1], lo[2 * R + 1];
     for (int k = -R; k <= R; k++) tot += g[k + R] = std::exp(-(double)k * k / (2.0 * kSigma[sig] * kSigma[sig]));
@@ -628,15 +634,14 @@ void fill(StripTables& T, int sig) {
         const __half a = __float2half_rn(x), b = __float2half_rn(x - __half2float(a));
         hi[k] = __half_raw(a).x;
         lo[k] = __half_raw(b).x;
-        T.taps[sig].g[k] = (__half2float(a) + __half2float(b)) / kTapScale;
-        T.taps[sig].cum[k] = (float)run;
+        T.cum[k] = (float)run;
         run += ((double)__half2float(a) + (double)__half2float(b)) / kTapScale;
     }
-    T.taps[sig].cum[2 * R + 1] = (float)run;
+    T.cum[2 * R + 1] = (float)run;
     auto put = [&](int op, int lane, int e, int k) {
         if (k < 0 || k > 2 * R) return;
-        T.op[sig][op][0][lane][e / 2] |= (uint32_t)hi[k] << (16 * (e & 1));
-        T.op[sig][op][1][lane][e / 2] |= (uint32_t)lo[k] << (16 * (e & 1));
+        T.op[op][0][lane][e / 2] |= (uint32_t)hi[k] << (16 * (e & 1));
+        T.op[op][1][lane][e / 2] |= (uint32_t)lo[k] << (16 * (e & 1));
     };
     for (int lane = 0; lane < 64; lane++)
         for (int e = 0; e < 8; e++) {
@@ -650,11 +655,10 @@ void fill(StripTables& T, int sig) {
 
 void fill_strip_tables(StripTables& T) {
     std::memset(&T, 0, sizeof(T));
-    fill<8>(T, SG_OPSIN);
-    fill<8>(T, SG_HIGH);
-    fill<8>(T, SG_MASK);
-    fill<9>(T, SG_MID);
-    fill<21>(T, SG_LOW);
+    fill<OpsinStage::R>(T.opsin, SG_OPSIN);
+    fill<LowStage::R>(T.low, SG_LOW);
+    fill<MidStage::R>(T.mid, SG_MID);
+    fill<HighStage::R>(T.high, SG_HIGH);
 }
 
 int strip_height(int w0, int h0, int w1, int h1, int npairs) {

@@ -26,10 +26,14 @@ enum : int {
 };
 static_assert(Q_T == Q_DB + 1 && Q_HFR == Q_T + 5 && Q_COUNT <= P_ACS, "plane layout");
 
+// Tables of the four stages' blurs.
 constexpr int kStripOps = 4;
 struct StripTables {
-    uint32_t op[kSigmaCount][kStripOps][2][64][4];  // tap operands: [h, l][lane][8 fp16]
-    Taps taps[kSigmaCount];                         // the taps as the operands represent them
+    struct alignas(16) Blur {
+        uint32_t op[kStripOps][2][64][4];  // tap operands: [h, l][lane][8 fp16]
+        float cum[44];                     // sums of the taps as the operands represent them, as in Taps
+    };
+    Blur opsin, low, mid, high;
 };
 void fill_strip_tables(StripTables& T);
 

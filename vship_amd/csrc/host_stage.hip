@@ -151,14 +151,6 @@ void HostStager::release() {
     pool_ = nullptr;
 }
 
-void HostStager::upload(void* dst, const void* src, size_t bytes, hipStream_t st) {
-    if (bytes == 0) return;
-    if (!dst || !src) VSHIP_THROW(E_BadPointer);
-    const uint8_t* s = static_cast<const uint8_t*>(src);
-    const UploadPlan P = plan_upload(&s, &bytes, 1);
-    upload(static_cast<uint8_t*>(dst), P, st);
-}
-
 void HostStager::upload(uint8_t* dst_base, const UploadPlan& plan, hipStream_t st) {
     if (!dst_base) VSHIP_THROW(E_BadPointer);
     if (shared_) return upload_shared(dst_base, plan, st);
@@ -249,7 +241,7 @@ void HostStager::upload_shared(uint8_t* dst_base, const UploadPlan& plan, hipStr
     team.run(
         pieces, n, nslots,
         [&](int c, bool wait) {
-            // the slot's previous DMA has to have read it before it is refilled
+            // the slot's previous move has to have read it before it is refilled
             hipEvent_t e = ev_[(first + c) % nslots];
             if (!wait) return hipEventQuery(e) == hipSuccess;
             HIP_OR_THROW(hipEventSynchronize(e), E_BadDeviceCode);

@@ -1,14 +1,16 @@
-// Host-to-device uploads through a ring of page-locked chunks.
+// Copies between the caller's memory and the device through a ring of
+// page-locked chunks.
 //
 // A copy from pageable memory has to pass through page-locked memory before
-// the DMA engine can read it. HostStager owns that memory: a ring of `slots`
+// the GPU can read it. HostStager owns that memory: a ring of `slots`
 // page-locked chunks with one event each. upload() copies a chunk of the
-// caller's bytes into the next free slot on the CPU (split over `threads`
-// threads), enqueues the slot's DMA on the given stream and records the
+// caller's bytes into the next free slot on the CPU (split over threads),
+// enqueues the slot's move to the device on the given stream and records the
 // slot's event, so that the CPU copy of chunk k+1 runs while chunk k crosses
-// PCIe, and a slot is refilled only after its DMA has finished. A source that
-// is already page-locked (hipHostMalloc) is handed to one DMA directly, and
-// upload() returns at once.
+// PCIe, and a slot is refilled only after its move has finished. A stager with
+// threads of its own moves its chunks by DMA, one without by a kernel or by DMA
+// (host_stage.hip says when). A source that is already page-locked
+// (hipHostMalloc) is handed to one DMA directly.
 //
 // One stager serves one caller thread at a time.
 #pragma once
@@ -62,22 +64,17 @@ public:
     HostStager(const HostStager&) = delete;
     HostStager& operator=(const HostStager&) = delete;
 
-    // Copies `bytes` from host `src` to device `dst`, in stream order on `st`.
-    // Returns once the caller's memory may be reused: at once for a
-    // page-locked source, after the last chunk has been copied into the ring
-    // otherwise. The DMA itself completes in stream order.
-    void upload(void* dst, const void* src, size_t bytes, hipStream_t st);
     // Uploads the runs of `plan` to dst_base + their offsets, in stream order
     // on `st`: page-locked runs by one DMA each, pageable runs packed in
     // device order into the ring's chunks (a chunk carries as many runs as
-    // fit, copied by the CPU threads, then one DMA). Returns once the callers'
-    // memory may be reused.
+    // fit, copied by the CPU threads, then moved in one piece). Returns once
+    // pageable memory may be reused; page-locked memory is read in stream order.
     void upload(uint8_t* dst_base, const UploadPlan& plan, hipStream_t st);
     // Copies `rows` rows of `row_bytes` bytes from device `src` (pitch
     // `src_stride`) to host `dst` (pitch `dst_stride`) after the work already
     // on `st`, and returns when they have arrived. A page-locked destination
     // takes one 2-D DMA; a pageable one receives the rows chunk by chunk from
-    // the ring, each chunk's DMA running while the previous one is copied out.
+    // the ring, one chunk arriving while the previous one is copied out.
     void download_rows(void* dst, int64_t dst_stride, const void* src, int64_t src_stride, size_t row_bytes,
                        int rows, hipStream_t st);
 
@@ -93,7 +90,7 @@ private:
 
     size_t chunk_ = 0;
     std::vector<uint8_t*> ring_;  // page-locked chunks
-    std::vector<hipEvent_t> ev_;  // slot i's last DMA
+    std::vector<hipEvent_t> ev_;  // slot i's last move
     int next_ = 0;
     ParallelCopy* pool_ = nullptr;
     bool shared_ = false;
