@@ -31,6 +31,13 @@ double wall_ms() {
     return duration<double, std::milli>(steady_clock::now().time_since_epoch()).count();
 }
 
+// Work ahead of a candidate's timed passes. The engine before it was freed and
+// its own allocated with the GPU idle, after which a pass takes 5 to 20 % longer
+// and gets shorter over some 30 ms (64 uneven pairs: 4.35, 4.06, 3.86, 3.76 ms,
+// from the eighth pass on 3.6): more than the candidates differ, so that one pass
+// of warm-up let a slower one win now and then (3.75 ms a pass instead of 3.57).
+constexpr double kWarmUpMs = 30.0;
+
 }  // namespace
 
 int size_class(int w, int h) {
@@ -122,8 +129,11 @@ Vship_Exception Vship_SSIMU2BatchTune(const Vship_SSIMU2Pair* pairs, int npairs,
                     o.persistent_grid = grids[gi];
                     o.use_graph = graph != 0;
                     Engine e(o);
-                    e.submit(in.data(), npairs);  // warm-up (and graph capture)
-                    e.wait(nullptr, nullptr);
+                    const double start = wall_ms();
+                    do {  // warm-up (and graph capture)
+                        e.submit(in.data(), npairs);
+                        e.wait(nullptr, nullptr);
+                    } while (wall_ms() - start < kWarmUpMs);
                     float best = 1e30f;
                     for (int r = 0; r < std::max(1, repeats); r++) {
                         const double t0 = wall_ms();
