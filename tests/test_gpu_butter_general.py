@@ -128,3 +128,13 @@ def test_the_strips_leave_far_pairs_out():
         best.append(min(t))
     say(f"  {best[0] * 1e6:.0f} us, far pairs {best[1] * 1e6:.0f} us")
     assert best[1] < 2.0 * best[0]
+
+
+@pytest.mark.parametrize("fmt", [api.PF_RGB_F32, api.PF_RGB_F16])
+def test_nan_samples_count_as_zero(fmt):
+    """A NaN sample linearises to 0, in the strips' range like any other."""
+    say("case NaN sample")
+    nan, zero = (norms_and_maps([far_pair(70, 50, 5, v, fmt)], 2, fmt) for v in (np.nan, 0.0))
+    assert np.isfinite(zero[0]).all()
+    assert np.array_equal(nan[0], zero[0])
+    assert np.array_equal(nan[1][0], zero[1][0])
