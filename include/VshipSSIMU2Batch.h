@@ -141,7 +141,8 @@ typedef struct {
     float map_ms;       /* blur + SSIM/edge maps, both precision classes */
     float map_fp32_ms;  /* map kernel of the segments with FP32 moment accumulation */
     float map_fp64_ms;  /* map kernel of the small segments (FP64 moment accumulation); about 0 where they
-                           ride along with the matrix-core kernel (an eager launch of one workgroup per tile) */
+                           ride along with the matrix-core kernel (persistent_grid 0, no graph, and fewer
+                           than four tiles per CU in its launch: one to three 1920x1080 pairs) */
     float finalize_ms;  /* FP64 norms + score kernel */
     float total_ms;     /* whole batch, first copy to last copy */
     int npairs;

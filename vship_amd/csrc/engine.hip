@@ -409,7 +409,8 @@ void launch_batch(const DescView& d, const PlanInfo& P, const LaunchShape& S, vo
                     const MapSplit M = map_split(tiles, eager, S.num_cus);
                     const int nsmall = eager && M.rows == 2 && tiles > 0 ? small[half] : 0;
                     if (!graph && tiles == 0) continue;
-                    const int grid = grid_for(tiles * M.csplit, 2 * fixed, 2 * fixed);
+                    const int twice = (int)std::min<int64_t>(2ll * fixed, INT32_MAX);  // half the waves each
+                    const int grid = grid_for(tiles * M.csplit, twice, twice);
                     HIP_OR_THROW(launch_map_mx(half, exact, M.rows, grid, nsmall, d.pairs, d.order_seg, d.order_start,
                                                d.hdr, arena, partials, M.csplit, st),
                                  E_BadDeviceCode);
