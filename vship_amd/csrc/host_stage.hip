@@ -90,12 +90,15 @@ std::shared_ptr<CopyTeam> shared_team() {
 // stream itself: a DMA and its hand-over to the kernels behind it cost about
 // 20 us each besides the bytes (measured at 1, 2 and 4 MiB), more than a small
 // picture's whole upload. Bound by PCIe; 64 workgroups keep 256 KiB of 16-byte
-// accesses in flight, several times what the link's latency needs. A copy that
-// finds the helpers taken, as most do where several handles work at once, takes
-// the DMA engines instead: there the link is never idle, and the kernel would
-// only wait for CUs behind the other handles' kernels and hold them up. 1920 x
-// 1080 float Butteraugli with its map, per call: one handle 1,765 us by the
-// kernel and 1,975 by DMA, eight handles on eight threads 1,110 and 965.
+// accesses in flight, several times what the link's latency needs. Where several
+// Butteraugli handles work at once, one that finds the helpers taken, as most do,
+// uses the DMA engines instead: the link is never idle there, and the kernel would
+// wait for CUs behind the other handles' stages (300 us of them per 1080p pair)
+// and hold them up. 1920 x 1080 float pairs with maps, per call: one handle
+// 1,765 us by the kernel and 1,975 by DMA, eight handles on eight threads 1,150
+// and 1,025. SSIMULACRA2's kernels are done in 75 us: eight threads 923 by the
+// kernel and 904 by DMA, but eight streams of the video filter 940 and 910 pairs/s,
+// so its handles stay with the kernel.
 constexpr int kMoveGroups = 64;
 __global__ __launch_bounds__(256) void move_kernel(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src,
                                                    size_t bytes) {
@@ -117,7 +120,8 @@ constexpr size_t kSharedMin = 1 << 20;   // below it, waking the helpers costs m
 
 }  // namespace
 
-HostStager::HostStager(int device, size_t chunk_bytes, int slots, int threads) : shared_(threads == 0) {
+HostStager::HostStager(int device, size_t chunk_bytes, int slots, int threads, bool dma_when_taken)
+    : shared_(threads == 0), dma_when_taken_(dma_when_taken) {
     HIP_OR_THROW(hipSetDevice(device), E_BadDeviceArgument);
     chunk_ = std::max<size_t>(chunk_bytes / 4096 * 4096, 4096);
     slots = std::max(slots, 2);
@@ -237,7 +241,7 @@ void HostStager::upload_shared(uint8_t* dst_base, const UploadPlan& plan, hipStr
     const int nslots = (int)ring_.size(), n = (int)chunks.size(), first = next_;
     next_ = (first + n) % nslots;
     CopyTeam& team = team_for(plan.total);
-    const bool dma = team.taken();
+    const bool dma = dma_when_taken_ && team.taken();
     team.run(
         pieces, n, nslots,
         [&](int c, bool wait) {
@@ -284,7 +288,7 @@ void HostStager::download_rows(void* dst, int64_t dst_stride, const void* src, i
     const int nchunks = (rows + per - 1) / per;
     const int nslots = (int)ring_.size();
     CopyTeam& team = team_for(row_bytes * rows);
-    const bool dma = !shared_ || team.taken();
+    const bool dma = !shared_ || (dma_when_taken_ && team.taken());
     // chunk c goes through slot (next_ + c) % nslots; up to nslots ahead
     auto enqueue = [&](int c) {
         const int k = (next_ + c) % nslots;

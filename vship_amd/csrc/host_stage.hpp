@@ -58,8 +58,9 @@ class HostStager {
 public:
     // threads: the CPU threads that copy pageable memory, the caller among them;
     // 0: the caller and, where they are free, the helpers that all such stagers
-    // of the process share (kept while one of them exists)
-    HostStager(int device, size_t chunk_bytes, int slots, int threads);
+    // of the process share (kept while one of them exists). dma_when_taken: its
+    // chunks go by DMA while another copy has the helpers.
+    HostStager(int device, size_t chunk_bytes, int slots, int threads, bool dma_when_taken = false);
     ~HostStager();
     HostStager(const HostStager&) = delete;
     HostStager& operator=(const HostStager&) = delete;
@@ -93,7 +94,7 @@ private:
     std::vector<hipEvent_t> ev_;  // slot i's last move
     int next_ = 0;
     ParallelCopy* pool_ = nullptr;
-    bool shared_ = false;
+    bool shared_ = false, dma_when_taken_ = false;
     std::shared_ptr<CopyTeam> team_;
     uint64_t pageable_bytes_ = 0, direct_bytes_ = 0;
 };

@@ -145,7 +145,7 @@ double FrameHandle::compute(int fmt, const uint8_t* const p1[3], const uint8_t* 
 // ---------------------------------------------------------------------------
 ButterHandle::ButterHandle(int w, int h, int qnorm, float intensity, int dev) : width(w), height(h), device(dev) {
     engine = std::make_unique<bt::Engine>(w, h, 1, qnorm, intensity, dev);
-    stager = std::make_unique<HostStager>(dev, (size_t)kFrameChunk, kFrameSlots, 0);
+    stager = std::make_unique<HostStager>(dev, (size_t)kFrameChunk, kFrameSlots, 0, true);
     HIP_OR_THROW(hipMalloc(reinterpret_cast<void**>(&map), sizeof(float) * (size_t)w * h), E_OutOfVRAM);
 }
 
