@@ -153,6 +153,8 @@ def per_frame_rate(descs, n, w, h, fp16):
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.json")
+TRAFFIC_SOURCE = ("profiles/hbm_traffic.json: rocprofv3 TCC_EA0_RDREQ_DRAM_32B + TCC_EA0_WRREQ_WRITE_DRAM_32B, "
+                  "x 32 bytes, per launch")
 VALU_FILE = os.path.join(ROOT, "profiles", "valu_issue.json")
 # MI355X vector ALUs: 256 CUs x 4 SIMDs x 16 lanes at the 2.4 GHz peak engine
 # clock; a wave64 VALU instruction is 64 lane-ops (4 cycles of its SIMD)
@@ -169,9 +171,10 @@ def _record(path, config, kernel):
 
 
 def measured_traffic(config, kernel):
-    """HBM bytes per launch of `kernel` on workload `config` from the committed
-    record of the FETCH_SIZE/WRITE_SIZE runs (calibrated on a device copy), or
-    None where no run of this kernel on this workload is recorded."""
+    """Bytes that one launch of `kernel` on workload `config` reads and writes
+    beyond the L2, from the committed record of the counter runs (requests in
+    units of 32 bytes), or None where no run of this kernel on this workload is
+    recorded."""
     rec = _record(TRAFFIC_FILE, config, kernel)
     return None if rec is None else rec["traffic_bytes"]
 
@@ -224,12 +227,12 @@ def roofline(st, map_ms, prep_ms, fp16, config):
     out = {"bound": "valu" if valu else "hbm"}
     out.update(valu if valu else hbm)
     out.update({"traffic": traffic,
-                "traffic_source": ("profiles/hbm_traffic.json: rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 per launch"
-                                   if traffic is not None else "no PMC run of this kernel on this workload"),
+                "traffic_source": (TRAFFIC_SOURCE if traffic is not None else "no PMC run of this kernel on this workload"),
                 "kernel": label, "hbm": hbm,
                 "algorithmic_bytes_per_launch": st["map_bytes_fp32"],
                 "note": f"2 images x 3 XYB planes x {elem} read per pixel of every scale in the FP32 class; "
-                        "the kernel is bound by vector-ALU issue (operand splitting and the maps), not HBM"})
+                        "the kernel is bound by vector-ALU issue (operand splitting and the maps) and, next to it, "
+                        "by its reads beyond the L2 (traffic)"})
     if valu:
         out["valu_source"] = "profiles/valu_issue.json: rocprofv3 SQ_INSTS_VALU minus SQ_INSTS_VALU_MFMA_F16 per " \
                              "launch over the live HIP-event duration"
@@ -469,8 +472,7 @@ def run_butter(a):
     traffic = measured_traffic(a.config, kernel)
     out["roofline"] = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                        "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                       "traffic_source": ("profiles/hbm_traffic.json: rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 "
-                                          "per launch" if traffic is not None
+                       "traffic_source": (TRAFFIC_SOURCE if traffic is not None
                                           else "no PMC run of this kernel on this workload"),
                        "kernel": f"{kernel} (both scales, {top} stage)",
                        "algorithmic_bytes_per_launch": int(stage_bytes[top]),

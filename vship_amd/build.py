@@ -30,9 +30,10 @@ HIPFLAGS = [
     "-I", os.path.join(ROOT, "include"),
 ]
 # Per-source options. The matrix-core map kernel is scheduled by LLVM's
-# iterative ILP strategy: 240 pairs of 1920x1080 in 11.09 ms, against 11.12 with
-# the memory-clause strategy, 11.15 with the default and 11.20 with the plain
-# ILP one, the same scores; 24 4K pairs 3.60, 3.64, 3.66 and 3.63.
+# iterative ILP strategy: 240 pairs of 1920x1080 in 10.81 to 10.82 ms, against
+# 10.88 to 10.89 with the memory-clause strategy and 10.92 to 10.93 with the
+# default (two alternating runs each, in which one side differs by 0.2 to 0.3 %;
+# 32 uneven pairs gain 0.3 to 1.7 %, eight 4:2:2 ones 0.8 to 1.3 %), the same scores.
 SOURCE_FLAGS = {
     "map_mfma.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
 }

@@ -3,7 +3,9 @@
 // The metric is the reference's src/butter/ (main.hpp:22-195): linear RGB at
 // full and half scale, opsin dynamics, four frequency bands, Malta line
 // differences, L2 terms, a psycho-visual mask, a blend of the two scales and
-// three norms. The arithmetic is FP32, as there.
+// three norms. The arithmetic is FP32, as there, but for the operands of the
+// matrix-core blurs, which are pairs of fp16 parts (23 significant bits;
+// butter_strip.hip says to what effect), and the norms, which are summed in FP64.
 //
 // Layout and kernels. Every intermediate is an FP32 plane in one arena, per
 // pair and scale: 47 planes of w x h (rows packed, planes 64-float aligned).
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(kThreads) void butter_input420_kernel(const PairDes
             }
             // each row's two pixels as one 8-byte store (xa is even and rows are
             // padded to 64 floats: with no second column, at an odd width, the
-            // second value lands in the row padding, which no kernel reads)
+            // second value lands in the row padding, whose values nothing uses)
             const int o0 = ya * S0.pitch + xa, o1 = yb * S0.pitch + xa, oh = (ya / 2) * S1.pitch + xa / 2;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
@@ -450,7 +452,9 @@ __device__ __forceinline__ RunPos run_pos() { return {(int)(threadIdx.x % kRuns)
 // The kRun values of a thread into a plane at row gy, columns gx .. gx + 7:
 // two 16-byte stores. gx is a multiple of 8 below the width and rows are
 // padded to a multiple of 64 floats, so the run stays inside its row; values
-// past the width land in the row padding, which no kernel reads.
+// past the width land in the row padding. The 16-byte loads of the strips and
+// of the Malta kernel read that padding and replace what they find by 0; no other
+// load reaches it.
 __device__ __forceinline__ void store_run(float* plane, int pitch, int gx, int gy, const float (&v)[kRun]) {
     float4* o = reinterpret_cast<float4*>(&at(plane, gy * pitch + gx));
     o[0] = make_float4(v[0], v[1], v[2], v[3]);

@@ -9,7 +9,9 @@
 // of another, so that the four SIMDs of a CU have the same work (a wave per
 // plane, five or six, left one or two of them with twice the others': sixteen
 // 1080p pairs took 0.68, 0.68 and 0.66 ms in the low, middle and opsin stages,
-// now 0.60, 0.58 and 0.57).
+// with halves 0.60, 0.58 and 0.57; with streaming stores and four opsin
+// workgroups per CU, see below, they take 0.56, 0.54 and 0.53, the high stage
+// 0.48).
 //
 //   row pass     Hr(16 rows x 16 cols) = In(16 x 32 input cols) . G(32 x 16)
 //   column pass  Out(16 rows x 16 cols) = G'(16 x 32 input rows) . Hr(32 x 16)
@@ -23,12 +25,18 @@
 // neighbouring pixels through the point operations.
 //
 // Operands are split into two fp16 parts x = h + l, both rounded to nearest,
-// and all four products accumulate in FP32. A value keeps 23 significant bits,
-// or an absolute error of 2^-25 where its low part is subnormal: linear RGB is
-// therefore stored times 2^10, and the taps carry 2^14. With h rounded towards
+// and all four products accumulate in FP32. A value keeps 23 significant bits of
+// FP32's 24, or an absolute error of 2^-25 where its low part is subnormal: linear
+// RGB is therefore stored times 2^10, and the taps carry 2^14. X and Y are
+// differences and sums of values above 1.7, whose own FP32 rounding is 2^-24, so
+// that 2^-25 is below what their planes hold, at any intensity. With h rounded towards
 // zero and without l l, whose parts then all have their values' sign, the norms
 // of 256 x 256 pairs were 0.65e-6 from their 64-bit values on average, now
-// 0.40e-6 (vector kernels 0.69e-6), for 0.5 % of the time of a batch. fp16 ends at 65,504, and inputs are not bounded by nature (float RGB;
+// 0.40e-6 (vector kernels 0.69e-6), for 0.5 % of the time of a batch. Maps of 60
+// pictures are 0.76e-6 of their mean from 64 bits on average (vector kernels
+// 1.20e-6), dark ones (samples below 0.08) 2.0e-5 (4.2e-5), at an intensity of 1
+// 0.92e-5 (1.84e-5), of a contrast of 0.02 3.9e-5 (6.4e-5).
+// fp16 ends at 65,504, and inputs are not bounded by nature (float RGB;
 // chroma far outside the gamut next to its opposite, at a high intensity):
 // the input kernels check float samples against kLinMax (those of the other
 // formats are below 10, of 32), and the opsin stage its results against kXybMax,
@@ -310,7 +318,9 @@ struct MidStage {
                 hx[im][k] = C.v[2 * im][k] - mf[2 * im][k];
                 const float yv = hy[im][k] = C.v[2 * im + 1][k] - mf[2 * im + 1][k];
                 const float s = 0.653020556257f, yw = 46.0f;
-                // hardware reciprocal (1 ulp) of a denominator of at least 46
+                // hardware reciprocal (1 ulp) of a denominator of at least 46: the
+                // general kernel divides, which gave maps and norms the same errors
+                // to three digits here and took the stage 5 of 545 us longer
                 hx[im][k] *= s + (yw * (1.0f - s)) * __builtin_amdgcn_rcpf(yw + yv * yv);
             }
             const float x0 = shrink(mf[0][k], 0.29f), x1 = shrink(mf[2][k], 0.29f);
@@ -615,8 +625,8 @@ void launch(const Scales& SS, int n, int th, const StripTables* tab, const Strip
                                       cdiv(SS.s[1].w, kStripW) * cdiv(SS.s[1].h, th));
     // Streaming stores where a stage writes more than the last-level cache
     // holds, so that the next stage would not find it there: sixteen 1080p
-    // pairs 0.60 -> 0.57 ms in the low stage (0.58 -> 0.55, 0.57 -> 0.56 and
-    // 0.50 -> 0.48 in the others), but one pair 42 -> 47 us.
+    // pairs 0.60 -> 0.57 ms in the low stage (0.58 -> 0.55 in the middle one, 0.57 ->
+    // 0.56 in opsin, 0.50 -> 0.48 in the high one), but one pair 42 -> 47 us.
     if ((int64_t)n * (SS.s[0].plane + SS.s[1].plane) * 5 * 4 > (int64_t)256 << 20)
         butter_strip_kernel<K, true><<<dim3((unsigned)wgs), dim3(kThreads), 0, st>>>(SS, n, th, tab, A);
     else
@@ -662,9 +672,9 @@ void fill_strip_tables(StripTables& T) {
 }
 
 int strip_height(int w0, int h0, int w1, int h1, int npairs) {
-    // As many workgroups as are resident at once (three per CU) while the
-    // picture gives them, then taller strips, whose first blocks (one to three,
-    // for the rows above) weigh less: sixteen 1080p pairs took 2.17 ms in the
+    // About as many workgroups as are resident at once (three per CU in the low and
+    // middle stages, four in the others) while the picture gives them, then taller
+    // strips, whose first blocks (one to three, for the rows above) weigh less: sixteen 1080p pairs took 2.17 ms in the
     // four stages at 128 rows and 2.12 ms at 256; one 1080p pair, and a 256 x 256
     // one, the same between 512 and 1,536 workgroups.
     int th = 16;

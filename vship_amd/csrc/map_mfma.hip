@@ -56,7 +56,9 @@
 // vector issue and 26 % with the matrix cores busy. Forms with fewer slots and more
 // products (28, 32) were no faster or slower, and 16 waves of this form per CU read
 // the centre samples from beyond the L2, at a lower clock, for no gain until those
-// came through LDS; twelve waves have the registers to load a window ahead.
+// came through LDS; twelve waves have the registers to load a window ahead. Memory
+// is the other bound by now: for 240 1080p pairs the kernel reads 32.4 GB beyond
+// the L2, where its planes hold 15.9 (a wave per strip read 18.4 GB), 4.8 TB/s.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -706,7 +708,8 @@ __device__ __forceinline__ void mx_tile(MxLds<SP::kParts, HS>& L, const TileGeo&
 }  // namespace
 
 // Occupancy: the two-part split fits 3 waves per SIMD (13.1 KB of LDS per wave,
-// under 170 VGPRs), the three-part split 2 (17.2 KB).
+// at most 168 VGPRs, none spilled), the three-part split 2 (17.2 KB). 46 to 61
+// SGPRs of either are kept in lanes of vector registers.
 //
 // HS: 1, a wave takes all rows of its 32 columns (workgroups of two waves); 2,
 // half of them (four waves, 80 input rows for 64 instead of 144 for 128), for

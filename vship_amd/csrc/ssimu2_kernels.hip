@@ -510,10 +510,11 @@ __device__ __forceinline__ void store_scale1(const PrepLds& L, const PairDev& P,
 // come from prep_quads, instantiated per input format; scales 2..5 go through
 // LDS. Every XYB plane is written exactly once. GEN = false takes the RGB and
 // staged 4:2:0 pairs, GEN = true the pairs of the generic chroma path; each
-// skips the other's tiles. Both are held to seven waves per SIMD (at most 72
-// VGPRs, no spills: the thread-index arithmetic is recomputed per use rather
-// than held across the tile loop, see tid_in_loop), which overlaps one
-// tile's stores with another's arithmetic.
+// skips the other's tiles. With QPT 4 both are held to seven waves per SIMD (at
+// most 72 VGPRs and none spilled, 8 or 9 SGPRs in the generic form: the
+// thread-index arithmetic is recomputed per use rather than held across the tile
+// loop, see tid_in_loop), which overlaps one tile's stores with another's
+// arithmetic.
 //
 // What bounds it is its writes (66 MB per 1080p pair, 3.30 ms for 240: 5.0 of the
 // 5.6 TB/s a write-only loop reaches) and vector issue (98 % of its cycles). Tiles
